@@ -1,6 +1,6 @@
-// SIMT slow path for the dtype pairs the matrix cores do not serve (int16/int32/int64/fp64 and
-// mixed pairs).  It restates the reference CPU backend's arithmetic exactly, one thread per
-// output element, reading operands through their strides:
+// SIMT path for the dtype pairs the matrix cores do not serve (int16/int32/int64 and mixed pairs;
+// fp64 with fp64 runs on gemm_f64.hip).  It restates the reference CPU backend's arithmetic exactly,
+// reading operands through their strides:
 //   * fp16/bf16 inputs are widened to fp32 first (src/backend/cpu/mul.cpp:110-111);
 //   * the result type is compute_type of the widened types (mul.cpp:112,
 //     include/core/type_traits.h:270-287);
@@ -21,6 +21,9 @@ template <> struct Promote<int8_t> { using type = int; };
 template <> struct Promote<int16_t> { using type = int; };
 template <typename A, typename B>
 using Common = decltype(typename Promote<A>::type{} + typename Promote<B>::type{});
+
+template <bool C, typename A, typename B> struct Pick { using type = A; };
+template <typename A, typename B> struct Pick<false, A, B> { using type = B; };
 
 template <typename X> struct Unsigned;
 template <> struct Unsigned<int8_t> { using type = uint8_t; };
@@ -72,17 +75,44 @@ template <typename Acc, typename P> __device__ inline Acc mac(Acc acc, P x, P y)
     return cvt<Acc>(add<Sum>((Sum)acc, (Sum)p));
 }
 
-// Load element `idx` of a tensor of storage dtype `dt` as compute type X (fp16/bf16 widened).
-template <typename X> __device__ inline X load_as(const void* p, int dt, int64_t idx) {
-    switch (dt) {
-        case TV_INT8: return cvt<X>(static_cast<const int8_t*>(p)[idx]);
-        case TV_INT16: return cvt<X>(static_cast<const int16_t*>(p)[idx]);
-        case TV_INT32: return cvt<X>(static_cast<const int32_t*>(p)[idx]);
-        case TV_INT64: return cvt<X>(static_cast<const long*>(p)[idx]);
-        case TV_BFLOAT16: return cvt<X>((float)static_cast<const __bf16*>(p)[idx]);
-        case TV_FLOAT16: return cvt<X>((float)static_cast<const _Float16*>(p)[idx]);
-        case TV_FLOAT32: return cvt<X>(static_cast<const float*>(p)[idx]);
-        default: return cvt<X>(static_cast<const double*>(p)[idx]);
+// Storage of an operand whose widened type is T: T itself, except that float also stands for fp16
+// and bf16 storage.  Raw<T> holds one element as loaded (16-bit elements zero-extended), so that a
+// batch of loads stays in flight until its elements are converted.
+template <typename T> struct RawOf { using type = T; };
+template <> struct RawOf<float> { using type = unsigned; };
+template <typename T> using Raw = typename RawOf<T>::type;
+
+// dst[e] = the element of storage type dt at ptr(e); one uniform branch for the whole batch.
+template <typename T, int N, class Ptr> __device__ inline void load_raw(int dt, Raw<T> (&dst)[N], const Ptr& ptr) {
+    if constexpr (__is_same(T, float)) {
+        if (dt == TV_FLOAT32) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) dst[e] = *reinterpret_cast<const unsigned*>(ptr(e));
+        } else {
+#pragma unroll
+            for (int e = 0; e < N; ++e) dst[e] = *reinterpret_cast<const unsigned short*>(ptr(e));
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) dst[e] = *reinterpret_cast<const T*>(ptr(e));
+    }
+}
+// put(e, widened element e) for a loaded batch.
+template <typename T, int N, class Put> __device__ inline void widen_raw(int dt, const Raw<T> (&src)[N], const Put& put) {
+    if constexpr (__is_same(T, float)) {
+        if (dt == TV_FLOAT32) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) put(e, __builtin_bit_cast(float, src[e]));
+        } else if (dt == TV_BFLOAT16) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) put(e, __builtin_bit_cast(float, src[e] << 16));
+        } else {
+#pragma unroll
+            for (int e = 0; e < N; ++e) put(e, (float)__builtin_bit_cast(_Float16, (unsigned short)src[e]));
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) put(e, src[e]);
     }
 }
 
@@ -97,49 +127,152 @@ template <typename S> __device__ inline void store_as(void* p, int dt, int64_t i
     }
 }
 
-template <int DT> struct CType;
-template <> struct CType<TV_INT8> { using type = int8_t; };
-template <> struct CType<TV_INT16> { using type = int16_t; };
-template <> struct CType<TV_INT32> { using type = int; };
-template <> struct CType<TV_INT64> { using type = long; };
-template <> struct CType<TV_FLOAT32> { using type = float; };
-template <> struct CType<TV_FLOAT64> { using type = double; };
+// Result type of the widened pair (T, R): compute_type (include/core/type_traits.h:270-287).
+template <typename T, typename R> constexpr auto result_value() {
+    if constexpr (__is_same(T, R)) return T{};
+    else if constexpr (is_int<T>() && is_int<R>()) {
+        if constexpr (sizeof(T) > sizeof(R)) return T{};
+        else return R{};
+    } else if constexpr (__is_same(T, double) || __is_same(R, double) || __is_same(T, long) || __is_same(R, long)) return double{};
+    else return float{};
+}
 
-// T, R: widened input types; S: result type.
-template <typename T, typename R, typename S>
-__global__ __launch_bounds__(256) void gemm_simt_kernel(GemmDesc d, int tiled) {
-    const int64_t total = (int64_t)d.batch * d.M * d.N;
-    for (int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; o < total; o += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t n = o % d.N;
-        const int64_t m = (o / d.N) % d.M;
-        const int64_t b = o / ((int64_t)d.N * d.M);
-        const int64_t ia = b * d.sa_b + m * d.sa_m;
-        const int64_t ib = b * d.sb_b + n * d.sb_n;
-        S res;
-        if (!tiled) {
-            using P = Common<T, R>;
-            P sum = 0;
-            for (int64_t k = 0; k < d.K; ++k) {
-                const P x = cvt<P>(load_as<T>(d.A, d.dtype_a, ia + k * d.sa_k));
-                const P y = cvt<P>(load_as<R>(d.B, d.dtype_b, ib + k * d.sb_k));
-                sum = mac<P, P>(sum, x, y);
-            }
-            res = cvt<S>(sum);
-        } else {
-            res = 0;
-            for (int64_t k0 = 0; k0 < d.K; k0 += 64) {
-                const int64_t k1 = k0 + 64 < d.K ? k0 + 64 : d.K;
-                T sum = 0;
-                for (int64_t k = k0; k < k1; ++k) {
-                    const T x = load_as<T>(d.A, d.dtype_a, ia + k * d.sa_k);
-                    const T y = cvt<T>(load_as<R>(d.B, d.dtype_b, ib + k * d.sb_k));
-                    sum = mac<T, T>(sum, x, y);
-                }
-                if (k0 == 0) res = cvt<S>(sum);
-                else res = cvt<S>(add<Common<S, S>>((Common<S, S>)res, (Common<S, S>)cvt<S>(sum)));
-            }
+// One workgroup computes 64 x 64 outputs, a thread 4 x 4 of them, summing k in order as the CPU
+// kernels do: every output's sum is the one thread's of a thread per output, bit for bit.  What
+// bounds the pairs is the VALU (fp32: one FMA per output and k; 32-bit integers: the quarter-rate
+// multiply), if operands are reused: with a thread per output, each multiply-add waited for two
+// loads from memory (0.3 us per k however small the call, 1.3 ms for 1000^3 in fp64).  Here 32 k of
+// both operands are converted once into LDS (two stages; the next 32 k are loaded into registers
+// while the current ones are multiplied, one barrier per 32 k), and a thread's 16 multiply-adds per
+// k read two 4-element vectors.  Against a thread per output, same box (us): fp32 x bf16
+// [1024,600]@[600,1024] 710 -> 47 (26 TFLOP/s), fp32 x fp16 [1000,600]@Wt[1000,600] 2390 -> 49,
+// int32 [1000,600]@[600,1000] 637 -> 55, int16 630 -> 53, fp32 x bf16 x[1,4096]@W[4096,4096]
+// 1753 -> 279, fp32 x fp16 [37,64]@[64,448] 21.4 -> 9.2.
+// X: the type the products run in: decltype(T + R), or T in the chunked sums (TILED).
+constexpr int kTile = 64, kBk = 32, kPitch = kTile + 4; // k rows of 64 elements, padded
+template <typename T, typename R, typename S, bool TILED>
+__global__ __launch_bounds__(256) void gemm_simt_kernel(GemmDesc d, int64_t tiles_m, int64_t tiles_n) {
+    using P = Common<T, R>;
+    using X = typename Pick<TILED, T, P>::type;
+    typedef X X4 __attribute__((ext_vector_type(4)));
+    static_assert(64 % kBk == 0, "a chunk is whole k-tiles");
+    __shared__ __attribute__((aligned(32))) X sa[2][kBk][kPitch];
+    __shared__ __attribute__((aligned(32))) X sb[2][kBk][kPitch];
+    constexpr int NE = kTile * kBk / 256; // elements per thread, operand and k-tile
+    const int tid = threadIdx.x;
+    const int tx = tid & 15, ty = tid >> 4;
+    // Consecutive threads along whichever dimension is contiguous: (row, k) of element e.
+    const bool ka = d.sa_k == 1, kb = d.sb_k == 1;
+    auto row_of = [&](bool kfast, int e) { return kfast ? (tid >> 5) + 8 * e : (tid & 63); };
+    auto k_of = [&](bool kfast, int e) { return kfast ? (tid & 31) : (tid >> 6) + 4 * e; };
+    const int64_t ntiles = tiles_m * tiles_n * d.batch;
+    const int nk = (d.K + kBk - 1) / kBk;
+    const int64_t esa = dtype_size(d.dtype_a), esb = dtype_size(d.dtype_b);
+
+    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        const int64_t b = t / (tiles_m * tiles_n), r = t - b * tiles_m * tiles_n;
+        const int64_t m0 = r / tiles_n * kTile, n0 = r % tiles_n * kTile;
+        Raw<T> ra[NE];
+        Raw<R> rb[NE];
+        // Element pointers at k-tile 0.  Rows past the matrix re-read its last row (their outputs are
+        // not stored); elements past K re-read k = 0 of the row and are not multiplied.
+        const char* pa[NE];
+        const char* pb[NE];
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            pa[e] = static_cast<const char*>(d.A) + (b * d.sa_b + min(m0 + row_of(ka, e), (int64_t)d.M - 1) * d.sa_m) * esa;
+            pb[e] = static_cast<const char*>(d.B) + (b * d.sb_b + min(n0 + row_of(kb, e), (int64_t)d.N - 1) * d.sb_n) * esb;
         }
-        store_as<S>(d.C, d.dtype_c, b * d.sc_b + m * d.sc_m + n * d.sc_n, res);
+        auto load = [&](int kt) {
+            load_raw<T>(d.dtype_a, ra, [&](int e) {
+                const int k = kt * kBk + k_of(ka, e);
+                return pa[e] + (k < d.K ? k : 0) * d.sa_k * esa;
+            });
+            load_raw<R>(d.dtype_b, rb, [&](int e) {
+                const int k = kt * kBk + k_of(kb, e);
+                return pb[e] + (k < d.K ? k : 0) * d.sb_k * esb;
+            });
+        };
+        auto store = [&](int st) {
+            widen_raw<T>(d.dtype_a, ra, [&](int e, T v) { sa[st][k_of(ka, e)][row_of(ka, e)] = cvt<X>(v); });
+            widen_raw<R>(d.dtype_b, rb, [&](int e, R v) { sb[st][k_of(kb, e)][row_of(kb, e)] = cvt<X>(v); });
+        };
+        X sum[4][4];
+        S res[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum[i][j] = 0, res[i][j] = 0;
+        auto read = [&](int st, int k, X4& x, X4& y) {
+            x = *reinterpret_cast<const X4*>(&sa[st][k][4 * ty]);
+            y = *reinterpret_cast<const X4*>(&sb[st][k][4 * tx]);
+        };
+        auto macs = [&](const X4& x, const X4& y) {
+            const X xs[4] = {x[0], x[1], x[2], x[3]}, ys[4] = {y[0], y[1], y[2], y[3]};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sum[i][j] = mac<X, X>(sum[i][j], xs[i], ys[j]);
+        };
+        if (nk > 0) {
+            load(0);
+            store(0);
+            load(1);
+        }
+        __syncthreads();
+        for (int kt = 0; kt < nk; ++kt) {
+            const int st = kt & 1;
+            store(st ^ 1); // read last in step kt - 1, before its barrier
+            load(kt + 2);
+            const int kn = min(kBk, d.K - kt * kBk);
+            if (kn == kBk) {
+                // The next G k's operands are read while the current G are multiplied: left to
+                // itself the compiler waited for each k's reads right after issuing them.
+                constexpr int G = sizeof(X) == 8 ? 2 : 4;
+                X4 x[2][G], y[2][G];
+#pragma unroll
+                for (int u = 0; u < G; ++u) read(st, u, x[0][u], y[0][u]);
+#pragma unroll
+                for (int g = 0; g < kBk / G; ++g) {
+                    if (g + 1 < kBk / G) {
+#pragma unroll
+                        for (int u = 0; u < G; ++u) read(st, (g + 1) * G + u, x[(g + 1) & 1][u], y[(g + 1) & 1][u]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int u = 0; u < G; ++u) macs(x[g & 1][u], y[g & 1][u]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                for (int k = 0; k < kn; ++k) {
+                    X4 x, y;
+                    read(st, k, x, y);
+                    macs(x, y);
+                }
+            }
+            if constexpr (TILED) {
+                if ((kt + 1) % (64 / kBk) == 0 || kt + 1 == nk) { // the end of a 64-wide chunk
+                    const bool first = (kt + 1) * kBk <= 64;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const S c = cvt<S>(sum[i][j]);
+                            res[i][j] = first ? c : cvt<S>(add<Common<S, S>>((Common<S, S>)res[i][j], (Common<S, S>)c));
+                            sum[i][j] = 0;
+                        }
+                }
+            }
+            __syncthreads();
+        }
+        S* C = static_cast<S*>(d.C) + b * d.sc_b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t m = m0 + 4 * ty + i, n = n0 + 4 * tx + j;
+                if (m < d.M && n < d.N) C[m * d.sc_m + n * d.sc_n] = TILED ? res[i][j] : cvt<S>(sum[i][j]);
+            }
     }
 }
 
@@ -147,31 +280,33 @@ static int widen(int dt) { return (dt == TV_BFLOAT16 || dt == TV_FLOAT16) ? TV_F
 
 template <typename T, typename R>
 static int launch_tr(const GemmDesc& d, hipStream_t stream) {
-    const int64_t total = (int64_t)d.batch * d.M * d.N;
-    const int tiled = total >= (int64_t)1024 * 1024;
-    int64_t blocks = (total + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    switch (d.dtype_c) {
-#define TV_S(DT)                                                                                                      \
-    case DT:                                                                                                          \
-        hipLaunchKernelGGL((gemm_simt_kernel<T, R, typename CType<DT>::type>), dim3((unsigned)blocks), dim3(256), 0, \
-                           stream, d, tiled);                                                                          \
-        return hipGetLastError();
-        TV_S(TV_INT8) TV_S(TV_INT16) TV_S(TV_INT32) TV_S(TV_INT64) TV_S(TV_FLOAT32) TV_S(TV_FLOAT64)
-#undef TV_S
-        default: return TV_E_DTYPE;
-    }
+    using S = decltype(result_value<T, R>());
+    const int64_t tiles_m = ((int64_t)d.M + kTile - 1) / kTile, tiles_n = ((int64_t)d.N + kTile - 1) / kTile;
+    // Up to 2^25 x 2^25 tiles and 2^31 batches: the grid is capped and a workgroup takes every
+    // grid-size-th tile; a count past 2^62 could never run.
+    const __int128 n = (__int128)tiles_m * tiles_n * d.batch;
+    if (n > ((__int128)1 << 62)) return TV_E_SHAPE;
+    const unsigned blocks = n < ((int64_t)1 << 20) ? (unsigned)n : 1u << 20;
+    if ((__int128)d.batch * d.M * d.N >= 1024 * 1024)
+        hipLaunchKernelGGL((gemm_simt_kernel<T, R, S, true>), dim3(blocks), dim3(256), 0, stream, d, tiles_m, tiles_n);
+    else
+        hipLaunchKernelGGL((gemm_simt_kernel<T, R, S, false>), dim3(blocks), dim3(256), 0, stream, d, tiles_m, tiles_n);
+    return hipGetLastError();
 }
 
 template <typename T>
 static int launch_t(const GemmDesc& d, hipStream_t stream) {
     switch (widen(d.dtype_b)) {
-        case TV_INT8: return launch_tr<T, int8_t>(d, stream);
+        case TV_INT8:
+            if constexpr (!__is_same(T, int8_t)) return launch_tr<T, int8_t>(d, stream);
+            else return TV_E_DTYPE; // int8 x int8 runs on the matrix cores
         case TV_INT16: return launch_tr<T, int16_t>(d, stream);
         case TV_INT32: return launch_tr<T, int>(d, stream);
         case TV_INT64: return launch_tr<T, long>(d, stream);
         case TV_FLOAT32: return launch_tr<T, float>(d, stream);
-        case TV_FLOAT64: return launch_tr<T, double>(d, stream);
+        case TV_FLOAT64:
+            if constexpr (!__is_same(T, double)) return launch_tr<T, double>(d, stream);
+            else return launch_gemm_f64(d, stream);
         default: return TV_E_DTYPE;
     }
 }
