@@ -91,13 +91,15 @@ struct DmaOperand {
     static constexpr int RB = ROWS * ES;           // M/N layout: bytes per k row
     static constexpr int CPR = RB / 16;            // M/N layout: chunks per k row
     static constexpr int KRB = 1024 / RB;          // M/N layout: k rows per block
-    // M/N layout: LDS bytes between the k-groups of a k-tile (64 int8 / 32 16-bit k rows) and
-    // between the two transposed reads of a fragment (8 / 4 k rows).
-    static constexpr int KGB = (ES == 1 ? 64 : 32) * RB;
-    static constexpr int RD2 = (ES == 1 ? 8 : 4) * RB;
+    // M/N layout: LDS bytes between the k-groups of a k-tile (64 int8 / 32 16-bit / 16 fp32 k rows)
+    // and between the two transposed reads of a fragment (8 / 4 k rows; fp32: between its four reads).
+    static constexpr int KGB = (64 / ES) * RB;
+    static constexpr int RD2 = (ES == 1 ? 8 : ES == 2 ? 4 : 1) * RB;
     static_assert(NBLK % NWAVES == 0, "load blocks must divide over the waves");
-    static_assert(MODE == LOAD_KCONTIG || (MODE == LOAD_MNCONTIG && ES <= 2 && (ROWS == 256 || ROWS == 128)),
-                  "M/N layout is laid out for 256- and 128-row int8 / 16-bit tiles");
+    static_assert(MODE == LOAD_KCONTIG || (MODE == LOAD_MNCONTIG && ((ES <= 2 && (ROWS == 256 || ROWS == 128)) ||
+                                                                     (ES == 2 && ROWS == 64) ||
+                                                                     (ES == 4 && (ROWS == 128 || ROWS == 64)))),
+                  "M/N layout: 256- and 128-row int8 / 16-bit tiles, 64-row 16-bit, 128- and 64-row fp32");
 
     const char* base; // element (row0, k = 0) of this tile, as bytes
     int64_t s_r, s_k; // element strides
@@ -112,8 +114,14 @@ struct DmaOperand {
     // distinct chunks among the 8 rows of each parity: (kr >> 1) & 3 and bit 4 of kr; it is the same
     // for the rows 8 and 64 apart that a lane's second read and k-group 1 read, and below 8, the
     // row's chunk count.
+    // 16-bit with 128-byte k rows (64-row tiles): again the row's parity picks the half; a pass reads
+    // 32 bytes of k rows r..r+3 and r+8..r+11, the two of each parity and block at distinct 32-byte
+    // pieces: bits 1 and 3 of kr.  fp32: a read takes 64 bytes of k rows e, e+4, e+8 and e+12, at
+    // distinct 64-byte pieces: bits 2 and 3 of kr.
     __device__ static inline int swz(int kr) {
-        if constexpr (ES == 1 && ROWS == 128) return ((kr >> 1) & 3) | (((kr >> 4) & 1) << 2);
+        if constexpr (ES == 4) return ((kr >> 2) & 3) << 2;
+        else if constexpr (ES == 2 && ROWS == 64) return (((kr >> 1) & 1) | (((kr >> 3) & 1) << 1)) << 1;
+        else if constexpr (ES == 1 && ROWS == 128) return ((kr >> 1) & 3) | (((kr >> 4) & 1) << 2);
         else if constexpr (ES == 1) return (kr & 7) | (((kr >> 4) & 1) << 3);
         else return ((kr & 3) | (((kr >> 3) & 1) << 2)) << 1;
     }
@@ -192,8 +200,10 @@ struct DmaOperand {
     //              address = (xf ^ (f << FSH)) + KGB kg + RD2 (second read).  A k row's bytes (RB,
     //              256 or 512) are a whole multiple of the 64 banks, so the swizzle spreads the
     //              rows of a transposed read over the banks the same way for either.
+    //  fp32 M/N layout: chunk (w0/4 + 4f + lane%16/4) ^ swz(kr), swz from the lane's group alone:
+    //              address = (xf ^ (f << 6)) + KGB kg + RB e for the fragment's four k rows e.
     unsigned xf;
-    static constexpr int FSH = ES == 1 ? 4 : 5;
+    static constexpr int FSH = ES == 1 ? 4 : ES == 2 ? 5 : 6;
     __device__ inline void xinit(unsigned op_base, int lane, int w0) {
         const int fr = lane & 15, grp = lane >> 4;
         if constexpr (MODE == LOAD_KCONTIG) {
@@ -201,6 +211,9 @@ struct DmaOperand {
         } else if constexpr (ES == 1) {
             const int kr = grp * 16 + (fr >> 1);
             xf = op_base + kr * RB + (fr & 1) * 8 + (((w0 / 16) ^ swz(kr)) << 4);
+        } else if constexpr (ES == 4) {
+            const int kr = grp * 4;
+            xf = op_base + kr * RB + (fr & 3) * 4 + (((w0 / 4 + (fr >> 2)) ^ swz(kr)) << 4);
         } else {
             const int kr = grp * 8 + (fr >> 2);
             const int c = fr & 3;
@@ -208,13 +221,19 @@ struct DmaOperand {
         }
     }
     // Fragment f of k-group kg in stage `st` (stage stride BYTES).
-    __device__ inline u32x4 frag_at(int st, int kg, int f) const {
+    __device__ inline u32x4 frag_at(int st, int kg, int f) const { return frag_from(xf, st * BYTES, kg, f); }
+    // The same from a base address: xf + the bytes of some stages, with `off` more bytes on top.
+    __device__ static inline u32x4 frag_from(unsigned xb, int off, int kg, int f) {
         if constexpr (MODE == LOAD_KCONTIG) {
-            const lds_char* p = (const lds_char*)(uintptr_t)(xf ^ (unsigned)(kg << 6)) + st * BYTES + f * 2048;
+            const lds_char* p = (const lds_char*)(uintptr_t)(xb ^ (unsigned)(kg << 6)) + off + f * 2048;
             return *(const __attribute__((address_space(3))) u32x4*)p;
         } else {
-            const lds_char* p = (const lds_char*)(uintptr_t)(xf ^ (unsigned)(f << FSH)) + st * BYTES + kg * KGB;
-            if constexpr (ES == 1) {
+            const lds_char* p = (const lds_char*)(uintptr_t)(xb ^ (unsigned)(f << FSH)) + off + kg * KGB;
+            if constexpr (ES == 4) {
+                typedef __attribute__((address_space(3))) unsigned lds_u32;
+                return u32x4{*(const lds_u32*)p, *(const lds_u32*)(p + RB), *(const lds_u32*)(p + 2 * RB),
+                             *(const lds_u32*)(p + 3 * RB)};
+            } else if constexpr (ES == 1) {
                 const i32x2_t a = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)p);
                 const i32x2_t b = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(p + RD2));
                 return u32x4{(unsigned)a.x, (unsigned)a.y, (unsigned)b.x, (unsigned)b.y};
@@ -283,7 +302,7 @@ struct DmaOperand {
         }
     }
 
-    static constexpr int kFragReads = MODE == LOAD_MNCONTIG ? 2 : 1;
+    static constexpr int kFragReads = MODE == LOAD_MNCONTIG ? (ES == 4 ? 4 : 2) : 1;
 };
 
 // int8 output of a whole BM x BN tile.  A wave's own block is 64-byte rows (half a cache line), so
@@ -298,7 +317,7 @@ __device__ inline void write_tile_wg_i8(const i32x4 (&acc)[C::FM][C::FN], char* 
     constexpr int NWAVES = C::THREADS / 64;
     constexpr int CPR = C::BN / 16;               // 16-byte chunks per tile row
     constexpr int RPW = C::BM / NWAVES;           // tile rows each wave stores
-    static_assert((RPW * CPR) % 64 == 0, "whole wave stores per row group");
+    static_assert((RPW * CPR) % 64 == 0 || RPW * CPR < 64, "whole wave stores per row group");
     // accumulators -> LDS: acc[i][j][q] is tile row wm*WM + 16i + lane%16, column
     // wn*WN + 16j + 4*(lane/16) + q; the 4 bytes of one (i, j) are one dword.
 #pragma unroll
@@ -314,15 +333,17 @@ __device__ inline void write_tile_wg_i8(const i32x4 (&acc)[C::FM][C::FN], char* 
         }
     lds_barrier();
 #pragma unroll
-    for (int it = 0; it < RPW * CPR / 64; ++it) {
+    for (int it = 0; it < (RPW * CPR + 63) / 64; ++it) {
         const int idx = it * 64 + lane;
+        if (RPW * CPR < 64 && idx >= RPW * CPR) break;
         const int r = wave * RPW + idx / CPR, c = idx % CPR;
         const u32x4 v = *reinterpret_cast<const u32x4*>(L + r * PITCH + c * 16);
         const int row = m0 + r, col = n0 + c * 16;
         if (row >= d.M) continue;
         int8_t* dst = reinterpret_cast<int8_t*>(Cb) + (int64_t)row * d.sc_m + col;
         if (col + 16 <= d.N) {
-            store_stream16(dst, v);
+            if constexpr (C::BN % 128 == 0) store_stream16(dst, v);
+            else *reinterpret_cast<u32x4*>(dst) = v; // part lines
         } else {
             const int8_t* e = reinterpret_cast<const int8_t*>(&v);
             for (int q = 0; q < 16 && col + q < d.N; ++q) dst[q] = e[q];
@@ -561,75 +582,6 @@ void gemm_dma_kernel(GemmDesc d, int tiles_m, int tiles_n, int group_m, int c_ve
         for (int j = 0; j < C::FN; ++j) acc[i][j] = Acc{0, 0, 0, 0};
     dma_tile_kloop<C>(d, L, b, m0, n0, 0, (d.K + C::BK - 1) / C::BK, acc);
     dma_tile_store<C, FUSED>(d, L, b, m0, n0, c_vec, acc);
-}
-
-// Stream-K schedule of the direct-load kernel, as gemm_mfma_sk_kernel (same iteration ranges, slots
-// and hand-over; int32 accumulators of int8 sum exactly in any order).
-template <class C, bool FUSED = false>
-__global__ __attribute__((amdgpu_flat_work_group_size(C::THREADS, C::THREADS),
-                          amdgpu_waves_per_eu(dma_waves_per_eu<C>(), dma_waves_per_eu<C>())))
-void gemm_dma_sk_kernel(GemmDesc d, int tiles_m, int tiles_n, int group_m, int c_vec, SkArgs sk) {
-    using Acc = typename Mfma<typename C::T>::Acc;
-    constexpr int SLOT = sk_slot_bytes<C>();
-    __shared__ __attribute__((aligned(1024))) char L[dma_lds_bytes<C>()];
-    __shared__ int last_flag;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int G = gridDim.x;
-    int w = blockIdx.x;
-    if ((G & 7) == 0) w = (w & 7) * (G >> 3) + (w >> 3);
-    const int64_t I = sk.iters;
-    const int nk = sk.nk;
-    const int64_t it_end = (int64_t)(w + 1) * I / G;
-    auto owner = [&](int64_t it) { return (int)(((it + 1) * G - 1) / I); };
-    auto slot_rsrc = [&](int slot) { return make_rsrc(sk.slots + (int64_t)slot * SLOT, SLOT); };
-
-    for (int64_t it = (int64_t)w * I / G; it < it_end;) {
-        const int tile = (int)(it / nk);
-        const int kt0 = (int)(it - (int64_t)tile * nk);
-        const int kt1 = (int)min((int64_t)nk, kt0 + (it_end - it));
-        it += kt1 - kt0;
-        int b, tm, tn;
-        mfma_tile_of(tile, tiles_m, tiles_n, group_m, b, tm, tn);
-        const int m0 = tm * C::BM, n0 = tn * C::BN;
-        Acc acc[C::FM][C::FN];
-#pragma unroll
-        for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-            for (int j = 0; j < C::FN; ++j) acc[i][j] = Acc{0, 0, 0, 0};
-        lds_barrier(); // the previous segment's epilogue is done with the LDS
-        dma_tile_kloop<C>(d, L, b, m0, n0, kt0, kt1, acc);
-        if (kt0 != 0 || kt1 != nk) {
-            const int64_t t0 = (int64_t)tile * nk;
-            const int first = owner(t0), last = owner(t0 + nk - 1);
-            {
-                const __amdgpu_buffer_rsrc_t r = slot_rsrc(w == first ? 2 * w + 1 : 2 * w);
-#pragma unroll
-                for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-                    for (int j = 0; j < C::FN; ++j)
-                        slot_store16(r, (((wave * C::FM + i) * C::FN + j) * 64 + lane) * 16, acc[i][j]);
-            }
-            publish_and_count(sk.cnt + tile, last - first + 1, &last_flag);
-            if (!last_flag) continue;
-            for (int v = first; v <= last; ++v) {
-                const __amdgpu_buffer_rsrc_t r = slot_rsrc(v == first ? 2 * v + 1 : 2 * v);
-#pragma unroll
-                for (int i = 0; i < C::FM; ++i) {
-#pragma unroll
-                    for (int j = 0; j < C::FN; ++j) {
-                        const Acc p = slot_load16<Acc>(r, (((wave * C::FM + i) * C::FN + j) * 64 + lane) * 16);
-                        acc[i][j] = v == first ? p : acc[i][j] + p;
-                    }
-                    // one row of slot loads at a time: with all of them hoisted, the loads and the
-                    // 128 accumulator registers exceed the 256 a wave has
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            slot_count_reset(sk.cnt + tile);
-        }
-        dma_tile_store<C, FUSED>(d, L, b, m0, n0, c_vec, acc);
-    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1163,66 +1115,8 @@ static int run_dma_chain(const GemmDesc& d, hipStream_t stream, int group_m, int
     return hipGetLastError();
 }
 
-// Stream-K launch of the direct-load kernel for few, long tiles: at most a quarter as many 256x256
-// tiles (half as many 128x128 tiles) as resident workgroups, and K of at least 64 k-tiles.  A split tile moves its fp32 partial sums
-// through the slots once per segment, which costs more than the balance gains once the tiles are
-// many.  Measured (settled clocks, same box, against one workgroup per tile) on int8 256x256 tiles
-// (one resident per CU): [512,8192]@[8192,8192] 52.0 against 75.5 us; and on bf16 256x256 tiles
-// before 16-bit GEMMs this small moved to 128x128 tiles: [512,8192]@[8192,8192] 88.9 against
-// 146.7 us, but 192 tiles (M = 3000, K = 4096) 121.5 against 83.0 us.  bf16 [128,8192]@[8192,8192]
-// (64 tiles of 128x128, two resident per CU) runs 43.5 us split.  c2 (256 tiles) and c3 (2048)
-// keep one workgroup per tile.  128x128 tiles split at up to half the resident workgroups: bf16
-// [512,8192]@[8192,8192] (256 tiles on 512 slots) 74.2 against 79.2 us, [1024,8192]@[8192,4096]
-// 74.5 against 80.1, [1024,4096]@[4096,4096] 43.0 against 45.1.  Returns 1 if it did not launch.
-template <class C, bool FUSED>
-static int run_dma_sk(const GemmDesc& d, hipStream_t stream, int group_m, int tiles_m, int tiles_n, int64_t ntiles, int c_vec) {
-    const int nk = (d.K + C::BK - 1) / C::BK;
-    if (nk < (__is_same(typename C::T, int8_t) ? 16 : 64)) return 1;
-    static std::atomic<int> grid[kMaxDevices];
-    int G = cached_per_device(grid, [](int dev) { return resident_grid(reinterpret_cast<const void*>(gemm_dma_sk_kernel<C, false>), C::THREADS, dev); });
-    if (G <= 0) return 1;
-    if (ntiles * (C::BM == 128 ? 2 : 4) > G) return 1;
-    // 16-bit 128x128 tiles above a quarter of the resident workgroups split only into segments of
-    // at least 32 k-tiles, or when the tile grid is one row or one column (each tile then streams
-    // its own rows of A or columns of B, HBM-bound, and the split adds streams).  Shorter segments
-    // of tiles whose operands are reused from L2 cost more in prologues and slot traffic than the
-    // idle CUs: bf16 [3000,4096]@[4096,1000] (192 tiles, 24 k-tiles per segment) 58.0 -> 47.3 us
-    // unsplit, [300,4096]@[4096,10000] 63.8 -> 59.2, [600,4096]@[4096,4096] 47.3 -> 43.0; but
-    // [8][3000,4096]@[4096,64] (192 tiles, one column each) 61.2 us split against 69.8,
-    // [300,4096]@[4096,4096] (96 tiles) 29.1 against 41.9, and [2048,8192]@[8192,2048] (256 tiles,
-    // 64 k-tiles per segment) 77.8 against 81.7.
-    if constexpr (!__is_same(typename C::T, int8_t) && C::BM == 128)
-        if (ntiles * 4 > G && tiles_m >= 2 && tiles_n >= 2 && ntiles * nk < 32 * (int64_t)G) return 1;
-    // int8 256x256 tiles split from 16 k-tiles (K >= 2048) when they are few (at most a fifth of
-    // the resident workgroups): one such tile takes a CU about 40 us at K = 4096, so a few of them
-    // leave the chip idle (int8 [512,4096]@[4096,4096] 41.0 -> 33.3 us, [256,4096]@[4096,4096]
-    // 40.5 -> 31.6, [16,4096]@[4096,4096] 40.2 -> 31.0); 64 tiles were slower split
-    // ([2048,2048]^3 24.2 against 28.5 us).  16-bit tiles split from 64 k-tiles.
-    if (nk < 64 && ntiles * 5 > G) return 1;
-    const int64_t iters = ntiles * nk;
-    if (iters / 8 < G) G = (int)(iters / 8);
-    // At most about four segments per tile, unless the segments stay at least 32 k-tiles long:
-    // bf16 [256,4096]@[4096,4096] (64 tiles of 128x128) 24.5 us in 4 against 32.0 in 8 and 28.7 in
-    // 2, [128,8192]@[8192,8192] 39.7 against 44.9 in 8; a single tile over K = 65536 keeps 32
-    // workgroups rather than 4.
-    const int64_t cap = 4 * ntiles > iters / 32 ? 4 * ntiles : iters / 32;
-    if (cap < G) G = (int)cap;
-    if (G < 1) return 1;
-    SkArgs sk;
-    sk.iters = iters;
-    sk.nk = nk;
-    sk.dp_tiles = 0; // every tile is split here (at most a quarter as many tiles as workgroups)
-    sk.wgs = G;
-    const int rc = gemm_sk_workspace(stream, (size_t)ntiles, (size_t)2 * G * sk_slot_bytes<C>(), &sk.cnt, &sk.slots);
-    if (rc == TV_E_NOMEM) return 1; // no room for the slots: one workgroup per tile serves the call
-    if (rc) return rc;
-    hipLaunchKernelGGL((gemm_dma_sk_kernel<C, FUSED>), dim3((unsigned)G), dim3(C::THREADS), 0, stream, d, tiles_m, tiles_n, group_m,
-                       c_vec, sk);
-    return hipGetLastError();
-}
-
 template <class C>
-static int run_dma_cfg(const GemmDesc& d, hipStream_t stream, int group_m, bool may_alloc) {
+static int run_dma_cfg(const GemmDesc& d, hipStream_t stream, int group_m) {
     const int tiles_m = (d.M + C::BM - 1) / C::BM;
     const int tiles_n = (d.N + C::BN - 1) / C::BN;
     const int64_t nwg = (int64_t)tiles_m * tiles_n * d.batch;
@@ -1238,17 +1132,6 @@ static int run_dma_cfg(const GemmDesc& d, hipStream_t stream, int group_m, bool 
     // The fused epilogue runs in the staged store only (16-byte aligned rows of C).
     const bool epi = d.bias != nullptr || d.act != TV_ACT_NONE;
     if (epi && d.sc_n != 1) return TV_E_UNSUPPORTED; // the fused store writes rows of C
-    if (may_alloc) {
-        // 16-bit GEMMs few enough to split (at most a quarter as many 256x256 tiles as CUs) always
-        // take 128x128 tiles in run_modes_dma, so the 256x256 16-bit configurations never split.
-        int rc = 1;
-        if constexpr (__is_same(typename C::T, int8_t))
-            rc = run_dma_sk<C, false>(d, stream, group_m, tiles_m, tiles_n, nwg, c_vec);
-        else if constexpr (C::BM == 128)
-            rc = epi ? run_dma_sk<C, true>(d, stream, group_m, tiles_m, tiles_n, nwg, c_vec)
-                     : run_dma_sk<C, false>(d, stream, group_m, tiles_m, tiles_n, nwg, c_vec);
-        if (rc != 1) return rc;
-    }
     if constexpr (!__is_same(typename C::T, int8_t) && C::BM == 256)
         if (!epi) {
             const int rc = run_dma_chain<C>(d, stream, group_m, tiles_m, tiles_n, nwg, c_vec);
@@ -1313,58 +1196,6 @@ static bool smallk_ok(const GemmDesc& d, int es, int bm_rows, int bn_rows) {
         return false;
     const int64_t tiles = (int64_t)((d.M + bm_rows - 1) / bm_rows) * ((d.N + bn_rows - 1) / bn_rows) * d.batch;
     return tiles >= 1024;
-}
-
-
-// 16-bit / int8 inputs: direct-to-LDS kernel for the vector layouts, gemm_mfma_kernel otherwise.
-template <typename T, int BM, int BN, int WMW, int WNW>
-static int run_modes_dma(const GemmDesc& d, hipStream_t stream, int group_m, bool may_alloc) {
-    const int es = (int)sizeof(T);
-    const int am = pick_mode(d.A, d.M, d.K, d.sa_m, d.sa_k, d.sa_b, d.batch, es, BM, d.pad_a);
-    const int bm = pick_mode(d.B, d.N, d.K, d.sb_n, d.sb_k, d.sb_b, d.batch, es, BN, d.pad_b);
-    // The small-K kernel has no fused epilogue (its staging area holds the output type only).
-    const bool epi = d.bias != nullptr || d.act != TV_ACT_NONE;
-    if (!epi && am != LOAD_GENERIC && bm != LOAD_GENERIC && smallk_ok(d, es, BM, BN)) {
-#define TV_CASE(A_, B_)                                                                                      \
-    if (am == A_ && bm == B_) {                                                                              \
-        if constexpr (sizeof(T) == 2) {                                                                      \
-            const int rc = run_smallk_pipe_cfg<GemmCfg<T, 128, 128, 2, 4, A_, B_>>(d, stream);               \
-            if (rc != 1) return rc;                                                                          \
-        }                                                                                                    \
-        return run_smallk_cfg<GemmCfg<T, BM, BN, WMW, WNW, A_, B_>>(d, stream);                              \
-    }
-        TV_CASE(LOAD_KCONTIG, LOAD_MNCONTIG)
-        TV_CASE(LOAD_KCONTIG, LOAD_KCONTIG)
-        TV_CASE(LOAD_MNCONTIG, LOAD_MNCONTIG)
-        TV_CASE(LOAD_MNCONTIG, LOAD_KCONTIG)
-#undef TV_CASE
-    }
-    // 16-bit and int8 GEMMs whose 128x128 tiles all fit one round of resident workgroups (two per
-    // CU) run 128x128 tiles: few 256x256 tiles leave CUs idle.  Measured against 256x256 tiles (and their
-    // stream-K schedule) on one box: bf16 [1024,4096]@[4096,4096] 45.5 against 62.7 us,
-    // [128,8192]@[8192,8192] 43.5 against 79.3, [2048]^3 25.6 against 41.6, [2048,4096]@[4096,4096]
-    // 67.4 against 78.6 (512 tiles of 128x128); but [3000,4096]@[4096,4096] (768 of them) 102.6
-    // against 83.7.
-    if constexpr (BM == 256 && BN == 256) {
-        const int64_t tiles128 = (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
-        if (am != LOAD_GENERIC && bm != LOAD_GENERIC && tiles128 <= 2 * (int64_t)device_cus()) {
-#define TV_CASE(A_, B_) \
-    if (am == A_ && bm == B_) return run_dma_cfg<GemmCfg<T, 128, 128, 2, 4, A_, B_>>(d, stream, group_m, may_alloc);
-            TV_CASE(LOAD_KCONTIG, LOAD_MNCONTIG)
-            TV_CASE(LOAD_KCONTIG, LOAD_KCONTIG)
-            TV_CASE(LOAD_MNCONTIG, LOAD_MNCONTIG)
-            TV_CASE(LOAD_MNCONTIG, LOAD_KCONTIG)
-#undef TV_CASE
-        }
-    }
-#define TV_CASE(A_, B_) \
-    if (am == A_ && bm == B_) return run_dma_cfg<GemmCfg<T, BM, BN, WMW, WNW, A_, B_>>(d, stream, group_m, may_alloc);
-    TV_CASE(LOAD_KCONTIG, LOAD_MNCONTIG)
-    TV_CASE(LOAD_KCONTIG, LOAD_KCONTIG)
-    TV_CASE(LOAD_MNCONTIG, LOAD_MNCONTIG)
-    TV_CASE(LOAD_MNCONTIG, LOAD_KCONTIG)
-#undef TV_CASE
-    return run_modes<T, BM, BN, WMW, WNW>(d, stream, group_m, may_alloc);
 }
 
 } // namespace tvk

@@ -1,5 +1,5 @@
 // float instantiation of the MFMA GEMM kernels (gemm_mfma_impl.h).
-#include "gemm_mfma_impl.h"
+#include "gemm_ms_impl.h"
 
 namespace tvk {
 // fp32 matrix cores are 16x slower than the 16-bit ones, so a tile's wasted rows and columns cost
@@ -43,7 +43,7 @@ bool f32_whole_rounds_256(const GemmDesc& d) {
     return tiles >= cus && tiles % cus == 0;
 }
 
-int pick_f32_tile(const GemmDesc& d) {
+int pick_f32_tile(const GemmDesc& d, double* us) {
     const int bm = f32_b_mode(d);
     const bool t96_ok = f32_a_mode_96(d) == LOAD_KCONTIG && (bm == LOAD_MNCONTIG || bm == LOAD_KCONTIG);
     int best = 0;
@@ -60,12 +60,46 @@ int pick_f32_tile(const GemmDesc& d) {
             best_cost = cost;
         }
     }
+    // The chosen tile's time: c1's rate, and what a launch costs beside it, more where few tiles are
+    // split between the workgroups (fp32 [1024]^3 37.9 us, [300,4096]@[4096,4096] 99.7 us).
+    const F32Tile& t = kF32Tiles[best];
+    const int64_t tiles = (int64_t)((d.M + t.bm - 1) / t.bm) * ((d.N + t.bn - 1) / t.bn) * d.batch;
+    *us = best_cost * d.K / 64.4e6 + (tiles < 512 ? 16.0 : 5.0);
     return best;
+}
+
+// Calls of few tiles run the multi-stage kernel on 64x64 or 32x64 tiles where that is cheaper: few
+// large tiles split over K leave their time in the hand-over.  fp32, us, tiles above -> multi-stage:
+// [1024]^3 37.9 -> 23.5, [1001,776]@[776,1004] 28 -> 20.5, [2574,1316]@Wt[1316,320] 40.7 -> 27.9,
+// [128,640]@Wt[640,1024] 13.2 -> 8.5, [512]^3 -> 9.3; [2592,2048]@[2048,4096] 343 against 347 there.
+// Prices as in gemm_ms_impl.h (32 k per k-tile; the matrix cores' time bounds these).
+constexpr MsTile kF32MsTiles[2] = {{32, 64, 3, 2.5, 2.0, 0.46, 0.94, 3.0, 0.25}, {64, 64, 3, 2.5, 2.6, 0.65, 1.65, 3.0, 0.25}};
+
+int run_f32_ms(const GemmDesc& d, hipStream_t stream, bool may_alloc, double other_us) { // 1: not cheaper
+    const int am = pick_mode(d.A, d.M, d.K, d.sa_m, d.sa_k, d.sa_b, d.batch, 4, 128, d.pad_a), bm = f32_b_mode(d);
+    if (am == LOAD_GENERIC || bm == LOAD_GENERIC) return 1;
+    const bool ok[2] = {am == LOAD_KCONTIG, true};
+    const MsPlan plan = ms_plan(d, (d.K + 31) / 32, kF32MsTiles, ok, 2, may_alloc);
+    if (plan.us >= other_us) return 1;
+#define TV_MS(TILE_, BM_, WM_, WN_, NST_, A_, B_) \
+    if (plan.tile == TILE_ && am == A_ && bm == B_) return run_ms_cfg<GemmCfg<float, BM_, 64, WM_, WN_, A_, B_>, NST_>(d, stream, plan);
+    TV_MS(0, 32, 1, 4, 4, LOAD_KCONTIG, LOAD_KCONTIG)
+    TV_MS(0, 32, 1, 4, 4, LOAD_KCONTIG, LOAD_MNCONTIG)
+    TV_MS(1, 64, 2, 2, 3, LOAD_KCONTIG, LOAD_KCONTIG)
+    TV_MS(1, 64, 2, 2, 3, LOAD_KCONTIG, LOAD_MNCONTIG)
+    TV_MS(1, 64, 2, 2, 3, LOAD_MNCONTIG, LOAD_KCONTIG)
+    TV_MS(1, 64, 2, 2, 3, LOAD_MNCONTIG, LOAD_MNCONTIG)
+#undef TV_MS
+    return 1;
 }
 } // namespace
 
 int launch_gemm_mfma_f32(const GemmDesc& d, hipStream_t stream, bool may_alloc) {
-    switch (pick_f32_tile(d)) {
+    double us = 0;
+    const int tile = pick_f32_tile(d, &us);
+    const int rc = run_f32_ms(d, stream, may_alloc, us);
+    if (rc != 1) return rc;
+    switch (tile) {
         case 0:
             if (f32_whole_rounds_256(d)) return run_modes<float, 256, 256, 2, 4>(d, stream, 8, may_alloc);
             return run_modes<float, 128, 128, 2, 2>(d, stream, 8, may_alloc);
