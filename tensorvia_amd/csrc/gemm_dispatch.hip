@@ -13,15 +13,16 @@ int launch_gemm_mfma_i8(const GemmDesc& d, hipStream_t stream, bool may_alloc);
 // vector loaders.  With a workspace, such an operand is copied once into rows of whole chunks, zero
 // past its valid extent (pad_a / pad_b tell the load-mode choice, and the matrix-core GEMV, that
 // the tail may be read), and the call runs on the copy.  Small calls keep the gather.
-static int pad_operand(GemmDesc& d, bool is_a, hipStream_t stream) {
+// Whether an operand gets one: *job is then its copy, and d points at it.
+static bool pad_operand(GemmDesc& d, bool is_a, hipStream_t stream, PadJob* job) {
     const int es = (int)dtype_size(is_a ? d.dtype_a : d.dtype_b);
-    if (es != 1 && es != 2 && es != 4) return 0;
+    if (es != 1 && es != 2 && es != 4) return false;
     const int64_t vec = 16 / es;
     const void* p = is_a ? d.A : d.B;
     const int64_t R = is_a ? d.M : d.N, K = d.K;
     const int64_t s_r = is_a ? d.sa_m : d.sb_n, s_k = is_a ? d.sa_k : d.sb_k, s_b = is_a ? d.sa_b : d.sb_b;
-    if (is_a ? d.pad_a : d.pad_b) return 0; // already a padded copy
-    if (pick_mode(p, R, K, s_r, s_k, s_b, d.batch, es, 256, false) != LOAD_GENERIC) return 0;
+    if (is_a ? d.pad_a : d.pad_b) return false; // already a padded copy
+    if (pick_mode(p, R, K, s_r, s_k, s_b, d.batch, es, 256, false) != LOAD_GENERIC) return false;
     int64_t L, rows, s_row;
     if (s_k == 1) { // rows (m / n) of L = K contiguous elements
         L = K;
@@ -32,19 +33,18 @@ static int pad_operand(GemmDesc& d, bool is_a, hipStream_t stream) {
         rows = K;
         s_row = s_k;
     } else {
-        return 0; // no contiguous dimension: the gather stays
+        return false; // no contiguous dimension: the gather stays
     }
-    if (L <= 0 || rows <= 0) return 0;
+    if (L <= 0 || rows <= 0) return false;
     const int64_t P = (L + vec - 1) / vec * vec;
     const int64_t nb = d.batch > 1 && s_b != 0 ? d.batch : 1;
     // The copy's layout must itself pass (a k-tile panel's offsets within 31 bits); nullptr stands
     // for the workspace's 16-byte aligned base.
     const int64_t ps_r = s_k == 1 ? P : 1, ps_k = s_k == 1 ? 1 : P, ps_b = nb > 1 ? rows * P : 0;
-    if (pick_mode(nullptr, R, K, ps_r, ps_k, ps_b, d.batch, es, 256, true) == LOAD_GENERIC) return 0;
+    if (pick_mode(nullptr, R, K, ps_r, ps_k, ps_b, d.batch, es, 256, true) == LOAD_GENERIC) return false;
     void* ws = nullptr;
-    if (gemm_pad_workspace(stream, (size_t)(nb * rows * P * es), is_a ? 0 : 1, &ws) != 0) return 0; // no room: gather
-    const int rc = launch_pad_rows(p, ws, es, nb, rows, s_row, s_b, L, P, stream);
-    if (rc) return rc;
+    if (gemm_pad_workspace(stream, (size_t)(nb * rows * P * es), is_a ? 0 : 1, &ws) != 0) return false; // no room: gather
+    *job = PadJob{p, ws, rows, nb * rows, s_row, s_b, L, P};
     if (is_a) {
         d.A = ws;
         (s_k == 1 ? d.sa_m : d.sa_k) = P;
@@ -56,7 +56,7 @@ static int pad_operand(GemmDesc& d, bool is_a, hipStream_t stream) {
         d.sb_b = nb > 1 ? rows * P : 0;
         d.pad_b = 1;
     }
-    return 0;
+    return true;
 }
 
 // Calls of at least this many multiply-adds, or of K at least kPadMinK, copy misaligned operands
@@ -68,8 +68,11 @@ constexpr int kPadMinK = 256;
 
 int pad_gemm_operands(GemmDesc& d, hipStream_t stream) {
     if ((int64_t)d.M * d.N * d.K * (d.batch > 1 ? d.batch : 1) < kPadMinMacs && d.K < kPadMinK) return 0;
-    const int rc = pad_operand(d, true, stream);
-    return rc ? rc : pad_operand(d, false, stream);
+    PadJob jobs[2];
+    int n = 0;
+    if (pad_operand(d, true, stream, &jobs[n])) ++n;
+    if (pad_operand(d, false, stream, &jobs[n])) ++n;
+    return n ? launch_pad_rows(jobs, n, (int)dtype_size(d.dtype_a), stream) : 0;
 }
 
 // The stride of a dimension of extent 1 (A's rows when M = 1, B's columns when N = 1, either

@@ -153,64 +153,70 @@ static int launch_transpose(const RepackDesc& r, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Zero-padded row copy of a GEMM operand (launch_gemm_mfma uses it for operands contiguous along
-// one dimension whose rows are not whole 16-byte chunks): destination row w = batch * rows + row
-// holds the source row's L elements, then zeros up to P.  One thread per 16-byte destination
-// chunk, consecutive threads on consecutive chunks (rows run on one after the other).  A chunk
-// wholly inside its row is read with the widest loads the row start's alignment allows (16, 8 or
-// 4 bytes; the same for every chunk of a row, since chunks are 16 bytes apart); a row's last,
-// partial chunk element by element.  IDX: 32-bit index arithmetic when the chunk count allows.
+// Zero-padded row copies of a GEMM's operands (pad_gemm_operands uses them for operands contiguous
+// along one dimension whose rows are not whole 16-byte chunks): destination row w = batch * rows + row
+// holds the source row's L elements, then zeros up to P.  One thread per 16-byte destination chunk,
+// consecutive threads on consecutive chunks (rows run on one after the other).  A chunk wholly inside
+// its row is one 16-byte load, at whatever alignment the row has (global loads here need none beyond
+// the byte): element by element, 16 loads per int8 chunk, the copy took longer than the product it
+// fed.  Both operands' copies are one launch,
+// the first `blocks_a` workgroups for the first: a launch more costs 3 to 4 us.
+// Whole calls, us: int8 [3,3695]@Wt[3695,2496] 24.0 -> 14.9, bf16 [2,2277]@Wt[2277,2238] 20.2 -> 15.7,
+// int8 [512,590]@Bt[590,448] 10.5 -> 7.4, bf16 [209,3794]@[3794,2284] 41.8 -> 37.0.
+// IDX: 32-bit index arithmetic when the chunk count allows.
 template <typename E, typename IDX>
-__global__ __launch_bounds__(256) void pad_rows_kernel(const E* src, E* dst, int64_t rows, int64_t nrows, int64_t s_row,
-                                                       int64_t s_batch, int64_t L, int64_t P) {
+__device__ inline void pad_rows(const PadJob& j, IDX first, IDX stride) {
     constexpr int V = 16 / (int)sizeof(E);
     struct Chunk {
         E e[V];
     };
-    const IDX cpr = (IDX)(P / V);
-    const IDX total = (IDX)nrows * cpr;
-    const IDX rws = (IDX)rows;
-    const IDX stride = (IDX)gridDim.x * blockDim.x;
-    for (IDX i = (IDX)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
+    const IDX cpr = (IDX)(j.P / V);
+    const IDX total = (IDX)j.nrows * cpr;
+    const IDX rws = (IDX)j.rows;
+    for (IDX i = first; i < total; i += stride) {
         const IDX w = i / cpr, c = i - w * cpr;
-        const IDX b = rws == (IDX)nrows ? 0 : w / rws, r = w - b * rws;
-        const E* s = src + (int64_t)b * s_batch + (int64_t)r * s_row;
+        const IDX b = rws == (IDX)j.nrows ? 0 : w / rws, r = w - b * rws;
+        const E* s = static_cast<const E*>(j.src) + (int64_t)b * j.s_batch + (int64_t)r * j.s_row;
         const int64_t x0 = (int64_t)c * V;
-        const char* q = reinterpret_cast<const char*>(s + x0);
-        const unsigned al = (unsigned)(reinterpret_cast<uintptr_t>(s) & 15);
         u32x4 v;
-        if (x0 + V <= L && al == 0) {
-            v = *reinterpret_cast<const u32x4*>(q);
-        } else if (x0 + V <= L && (al & 7) == 0) {
-            const uint2 lo = reinterpret_cast<const uint2*>(q)[0], hi = reinterpret_cast<const uint2*>(q)[1];
-            v = u32x4{lo.x, lo.y, hi.x, hi.y};
-        } else if (x0 + V <= L && (al & 3) == 0) {
-            const unsigned* u = reinterpret_cast<const unsigned*>(q);
-            v = u32x4{u[0], u[1], u[2], u[3]};
+        if (j.L >= V) { // uniform
+            // The row's last 16 bytes serve its partial chunk, shifted down (zeros follow).
+            const int64_t x = x0 + V <= j.L ? x0 : j.L - V;
+            unsigned __int128 q;
+            __builtin_memcpy(&q, reinterpret_cast<const char*>(s + x), 16);
+            q >>= (unsigned)(x0 - x) * 8 * (unsigned)sizeof(E);
+            v = __builtin_bit_cast(u32x4, q);
         } else {
             Chunk t;
 #pragma unroll
-            for (int e = 0; e < V; ++e) t.e[e] = x0 + e < L ? s[x0 + e] : E(0);
+            for (int e = 0; e < V; ++e) t.e[e] = x0 + e < j.L ? s[x0 + e] : E(0);
             v = __builtin_bit_cast(u32x4, t);
         }
-        *reinterpret_cast<u32x4*>(dst + (int64_t)w * P + x0) = v;
+        *reinterpret_cast<u32x4*>(static_cast<E*>(j.dst) + (int64_t)w * j.P + x0) = v;
     }
 }
+template <typename E, typename IDX>
+__global__ __launch_bounds__(256) void pad_rows_kernel(PadJob a, PadJob b, unsigned blocks_a) {
+    if (blockIdx.x < blocks_a) pad_rows<E, IDX>(a, (IDX)blockIdx.x * 256 + threadIdx.x, (IDX)blocks_a * 256);
+    else pad_rows<E, IDX>(b, (IDX)(blockIdx.x - blocks_a) * 256 + threadIdx.x, (IDX)(gridDim.x - blocks_a) * 256);
+}
 
-int launch_pad_rows(const void* src, void* dst, int es, int64_t nb, int64_t rows, int64_t s_row, int64_t s_batch, int64_t L,
-                    int64_t P, hipStream_t stream) {
-    const int64_t nrows = nb * rows;
-    if (nrows <= 0 || L <= 0 || P < L || (P * es) % 16 != 0) return TV_E_SHAPE;
-    const int64_t chunks = nrows * (P * es / 16);
-    const unsigned grid = grid_for(chunks, 256);
-    const bool small = chunks < ((int64_t)1 << 31);
+int launch_pad_rows(const PadJob* jobs, int n, int es, hipStream_t stream) {
+    if (n < 1 || n > 2) return TV_E_SHAPE;
+    unsigned blocks[2] = {0, 0};
+    bool small = true;
+    for (int i = 0; i < n; ++i) {
+        const PadJob& j = jobs[i];
+        if (j.nrows <= 0 || j.L <= 0 || j.P < j.L || (j.P * es) % 16 != 0) return TV_E_SHAPE;
+        const int64_t chunks = j.nrows * (j.P * es / 16);
+        blocks[i] = grid_for(chunks, 256);
+        small = small && chunks < ((int64_t)1 << 31);
+    }
+    const PadJob& b = jobs[n - 1];
+    const dim3 grid(blocks[0] + blocks[1]);
 #define TV_PAD(E)                                                                                                      \
-    if (small)                                                                                                         \
-        hipLaunchKernelGGL((pad_rows_kernel<E, uint32_t>), dim3(grid), dim3(256), 0, stream, static_cast<const E*>(src), \
-                           static_cast<E*>(dst), rows, nrows, s_row, s_batch, L, P);                                  \
-    else                                                                                                               \
-        hipLaunchKernelGGL((pad_rows_kernel<E, int64_t>), dim3(grid), dim3(256), 0, stream, static_cast<const E*>(src),  \
-                           static_cast<E*>(dst), rows, nrows, s_row, s_batch, L, P);
+    if (small) hipLaunchKernelGGL((pad_rows_kernel<E, uint32_t>), grid, dim3(256), 0, stream, jobs[0], b, blocks[0]);  \
+    else hipLaunchKernelGGL((pad_rows_kernel<E, int64_t>), grid, dim3(256), 0, stream, jobs[0], b, blocks[0]);
     switch (es) {
         case 1: TV_PAD(uint8_t) break;
         case 2: TV_PAD(uint16_t) break;

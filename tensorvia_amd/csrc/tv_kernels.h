@@ -220,11 +220,16 @@ int launch_gemv(const GemmDesc& d, hipStream_t stream, const GemvScratch* fixed 
 // The static split-K scratch of the current device (set up on its first use: its address is looked
 // up and its counters cleared on `stream`).
 int gemv_static_scratch(hipStream_t stream, GemvScratch* out);
-// Zero-padded row copy of a GEMM operand: nb batches (source stride s_batch) of `rows` rows (source
-// stride s_row) of L contiguous elements of `es` bytes, written densely as rows of P elements (P a
-// multiple of 16 bytes), zero in [L, P).
-int launch_pad_rows(const void* src, void* dst, int es, int64_t nb, int64_t rows, int64_t s_row, int64_t s_batch,
-                    int64_t L, int64_t P, hipStream_t stream);
+// Zero-padded row copy of a GEMM operand: nrows rows (`rows` per batch; source strides s_row and
+// s_batch, in elements) of L contiguous elements, written densely as rows of P elements (P a multiple
+// of 16 bytes), zero in [L, P).
+struct PadJob {
+    const void* src;
+    void* dst;
+    int64_t rows, nrows, s_row, s_batch, L, P;
+};
+// One or two such copies of `es`-byte elements in one launch.
+int launch_pad_rows(const PadJob* jobs, int n, int es, hipStream_t stream);
 // Per-(device, stream) buffer for the padded copy of operand A (operand 0) or B (operand 1).
 int gemm_pad_workspace(hipStream_t stream, size_t bytes, int operand, void** out);
 
