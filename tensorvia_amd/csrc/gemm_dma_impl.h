@@ -312,7 +312,7 @@ struct DmaOperand {
 // the k-loop's LDS free (after a workgroup barrier); L holds at least BM * (BN + 16) bytes.
 template <class C>
 __device__ inline void write_tile_wg_i8(const i32x4 (&acc)[C::FM][C::FN], char* L, char* Cb, int lane, int wave, int wm,
-                                        int wn, int m0, int n0, const GemmDesc& d) {
+                                        int wn, int m0, int n0, const GemmDesc& d, bool aligned) {
     constexpr int PITCH = C::BN + 16;
     constexpr int NWAVES = C::THREADS / 64;
     constexpr int CPR = C::BN / 16;               // 16-byte chunks per tile row
@@ -342,7 +342,8 @@ __device__ inline void write_tile_wg_i8(const i32x4 (&acc)[C::FM][C::FN], char* 
         if (row >= d.M) continue;
         int8_t* dst = reinterpret_cast<int8_t*>(Cb) + (int64_t)row * d.sc_m + col;
         if (col + 16 <= d.N) {
-            if constexpr (C::BN % 128 == 0) store_stream16(dst, v);
+            if (!aligned) __builtin_memcpy(dst, &v, 16);
+            else if constexpr (C::BN % 128 == 0) store_stream16(dst, v);
             else *reinterpret_cast<u32x4*>(dst) = v; // part lines
         } else {
             const int8_t* e = reinterpret_cast<const int8_t*>(&v);
@@ -513,52 +514,52 @@ __device__ __attribute__((always_inline)) inline void dma_tile_store(const GemmD
     // All waves leave the k-loop's LDS before any wave stages its output there (the barriers below).
     const size_t csz = dtype_size(d.dtype_c);
     char* Cb = static_cast<char*>(d.C) + (int64_t)b * d.sc_b * csz;
+    const bool aligned = c_vec == 2;
     if constexpr (FUSED && !__is_same(Acc, i32x4)) {
         // Fused epilogue: fp32 staging, bias and activation after the accumulators are dead.
         lds_barrier();
         char* lw = (wave < NWAVES / 2 ? S0 : S1) + (wave % (NWAVES / 2)) * EPI;
         const int mrow0 = m0 + wm * C::WM, ncol0 = n0 + wn * C::WN;
-        if (c_vec == 2 && (d.bias == nullptr || d.sbias_m == 0)) {
+        if (d.bias == nullptr || d.sbias_m == 0) {
             // per-column (or no) bias: applied as the accumulators are staged by the plain store
             auto store = [&](const auto& f) {
-                if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, f);
-                else if (d.dtype_c == TV_FLOAT16) write_tile_staged<_Float16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, f);
-                else write_tile_staged<float, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, f);
+                if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned, f);
+                else if (d.dtype_c == TV_FLOAT16) write_tile_staged<_Float16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned, f);
+                else write_tile_staged<float, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned, f);
             };
             if (d.act == TV_ACT_SILU || d.act == TV_ACT_SIGMOID || d.act == TV_ACT_TANH) store(ColBiasAct<C::FN, true>(d, b, ncol0, lane));
             else store(ColBiasAct<C::FN, false>(d, b, ncol0, lane));
             return;
         }
-        if (d.dtype_c == TV_BFLOAT16) write_tile_staged_epi<__bf16, C, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, b, c_vec != 0);
-        else if (d.dtype_c == TV_FLOAT16) write_tile_staged_epi<_Float16, C, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, b, c_vec != 0);
-        else write_tile_staged_epi<float, C, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, b, c_vec != 0);
+        if (d.dtype_c == TV_BFLOAT16) write_tile_staged_epi<__bf16, C, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, b, aligned);
+        else if (d.dtype_c == TV_FLOAT16) write_tile_staged_epi<_Float16, C, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, b, aligned);
+        else write_tile_staged_epi<float, C, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, b, aligned);
         return;
     }
-    if (c_vec == 2) {
+    if (c_vec != 0) {
         lds_barrier();
         char* lw = (wave < NWAVES / 2 ? S0 : S1) + (wave % (NWAVES / 2)) * EPI;
         const int mrow0 = m0 + wm * C::WM, ncol0 = n0 + wn * C::WN;
         if constexpr (__is_same(Acc, i32x4)) {
             static_assert(C::BM * (C::BN + 16) <= 2 * STAGE, "the int8 tile staging fits the k-loop's LDS");
-            if (d.dtype_c == TV_INT8) write_tile_wg_i8<C>(acc, L, Cb, lane, wave, wm, wn, m0, n0, d);
-            else write_tile_staged<int32_t, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d);
+            if (d.dtype_c == TV_INT8) write_tile_wg_i8<C>(acc, L, Cb, lane, wave, wm, wn, m0, n0, d, aligned);
+            else write_tile_staged<int32_t, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
         } else {
-            if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d);
-            else if (d.dtype_c == TV_FLOAT16) write_tile_staged<_Float16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d);
-            else write_tile_staged<float, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d);
+            if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
+            else if (d.dtype_c == TV_FLOAT16) write_tile_staged<_Float16, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
+            else write_tile_staged<float, C, Acc, EPI>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
         }
         return;
     }
     const int row0 = m0 + wm * C::WM + (lane & 15);
     const int col0 = n0 + wn * C::WN + (lane >> 4) * 4;
-    const bool vec_ok = c_vec != 0;
     if constexpr (__is_same(Acc, i32x4)) {
-        if (d.dtype_c == TV_INT8) write_tile<int8_t, C>(acc, Cb, row0, col0, vec_ok, d);
-        else write_tile<int32_t, C>(acc, Cb, row0, col0, vec_ok, d);
+        if (d.dtype_c == TV_INT8) write_tile<int8_t, C>(acc, Cb, row0, col0, d);
+        else write_tile<int32_t, C>(acc, Cb, row0, col0, d);
     } else {
-        if (d.dtype_c == TV_BFLOAT16) write_tile<__bf16, C>(acc, Cb, row0, col0, vec_ok, d);
-        else if (d.dtype_c == TV_FLOAT16) write_tile<_Float16, C>(acc, Cb, row0, col0, vec_ok, d);
-        else write_tile<float, C>(acc, Cb, row0, col0, vec_ok, d);
+        if (d.dtype_c == TV_BFLOAT16) write_tile<__bf16, C>(acc, Cb, row0, col0, d);
+        else if (d.dtype_c == TV_FLOAT16) write_tile<_Float16, C>(acc, Cb, row0, col0, d);
+        else write_tile<float, C>(acc, Cb, row0, col0, d);
     }
 }
 
@@ -1083,8 +1084,8 @@ void gemm_dma_chain_kernel(GemmDesc d, int tiles_m, int tiles_n, int group_m, in
         char* Cb = static_cast<char*>(d.C) + (int64_t)b * d.sc_b * (int64_t)dtype_size(d.dtype_c);
         char* lw = E + wave * EPI;
         const int ln = lane_here(), mrow0 = tm * C::BM + wm * C::WM, ncol0 = tn * C::BN + wn * C::WN;
-        if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C, Acc, EPI>(acc, lw, Cb, ln, mrow0, ncol0, d);
-        else write_tile_staged<_Float16, C, Acc, EPI>(acc, lw, Cb, ln, mrow0, ncol0, d);
+        if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C, Acc, EPI>(acc, lw, Cb, ln, mrow0, ncol0, d, true);
+        else write_tile_staged<_Float16, C, Acc, EPI>(acc, lw, Cb, ln, mrow0, ncol0, d, true);
         if (next >= hi) break;
         t = next;
     }
@@ -1122,14 +1123,8 @@ static int run_dma_cfg(const GemmDesc& d, hipStream_t stream, int group_m) {
     const int64_t nwg = (int64_t)tiles_m * tiles_n * d.batch;
     if (nwg <= 0) return 0;
     if (nwg > 0x7FFFFFFF) return TV_E_SHAPE;
-    const size_t csz = dtype_size(d.dtype_c);
-    int c_vec = d.sc_n == 1 && d.sc_m % 4 == 0 && (d.batch <= 1 || d.sc_b % 4 == 0) &&
-                (reinterpret_cast<uintptr_t>(d.C) % (4 * csz)) == 0;
-    const int64_t v16 = 16 / (int64_t)csz;
-    if (c_vec && d.sc_m % v16 == 0 && (d.batch <= 1 || d.sc_b % v16 == 0) &&
-        (reinterpret_cast<uintptr_t>(d.C) % 16) == 0 && (C::WN * (int64_t)csz) % 16 == 0)
-        c_vec = 2;
-    // The fused epilogue runs in the staged store only (16-byte aligned rows of C).
+    const int c_vec = c_store_mode(d);
+    // The fused epilogue runs in the staged store only.
     const bool epi = d.bias != nullptr || d.act != TV_ACT_NONE;
     if (epi && d.sc_n != 1) return TV_E_UNSUPPORTED; // the fused store writes rows of C
     if constexpr (!__is_same(typename C::T, int8_t) && C::BM == 256)

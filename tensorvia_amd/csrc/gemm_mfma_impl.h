@@ -279,32 +279,34 @@ struct GemmCfg {
 // wrap), the reference CPU backend's int8 result; half outputs round to nearest even.
 template <typename TC, typename V> __device__ inline TC cvt_out(V v) { return static_cast<TC>(v); }
 
-// Store the wave's accumulators as TC: acc[i][j][q] is C[row0 + 16i][col0 + 16j + q] (the lane's
-// row and first column are folded into row0 / col0), four consecutive columns per vector store.
+// Store the wave's accumulators as TC, element by element (column-strided C): acc[i][j][q] is
+// C[row0 + 16i][col0 + 16j + q] (the lane's row and first column are folded into row0 / col0).
 template <typename TC, class C, typename Acc>
-__device__ inline void write_tile(const Acc (&acc)[C::FM][C::FN], char* Cb, int row0, int col0, bool vec_ok,
-                                  const GemmDesc& d) {
-    typedef TC vec_t __attribute__((__vector_size__(4 * sizeof(TC))));
+__device__ inline void write_tile(const Acc (&acc)[C::FM][C::FN], char* Cb, int row0, int col0, const GemmDesc& d) {
 #pragma unroll
     for (int i = 0; i < C::FM; ++i) {
         const int row = row0 + 16 * i;
         if (row >= d.M) continue;
         TC* crow = reinterpret_cast<TC*>(Cb) + (int64_t)row * d.sc_m;
 #pragma unroll
-        for (int j = 0; j < C::FN; ++j) {
-            const int col = col0 + 16 * j;
-            if (vec_ok && col + 4 <= d.N) {
-                vec_t v;
+        for (int j = 0; j < C::FN; ++j)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] = cvt_out<TC>(acc[i][j][q]);
-                *reinterpret_cast<vec_t*>(crow + col) = v;
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (col + q < d.N) crow[(int64_t)(col + q) * d.sc_n] = cvt_out<TC>(acc[i][j][q]);
+            for (int q = 0; q < 4; ++q) {
+                const int col = col0 + 16 * j + q;
+                if (col < d.N) crow[(int64_t)col * d.sc_n] = cvt_out<TC>(acc[i][j][q]);
             }
-        }
     }
+}
+
+// How a kernel stores C (`c_vec`): element by element (0, column-strided C), or rows staged through
+// LDS and stored in 16-byte chunks, at whatever alignment the rows have (1) or all 16-byte aligned
+// (2).  Unaligned rows (an odd N) stored element by element from the accumulators' layout, 2 bytes of
+// 16 rows per instruction, took longer than the product: us, fp16 [16][1117,80]@Kt[80,1117] 43.2 -> 19.1,
+// bf16 [6][1952,524]@[524,2017] 82.1 -> 52.8, fp32 [1001,777]@[777,1003] 31.2 -> 28.1.
+inline int c_store_mode(const GemmDesc& d) {
+    const int64_t v16 = 16 / (int64_t)dtype_size(d.dtype_c);
+    if (d.sc_n != 1 && d.N > 1) return 0;
+    return (d.M <= 1 || d.sc_m % v16 == 0) && (d.batch <= 1 || d.sc_b % v16 == 0) && aligned16(d.C) ? 2 : 1;
 }
 
 // LDS bytes each wave gets for staging its output tile.
@@ -313,8 +315,8 @@ constexpr int kEpiWaveBytes = 18432;
 // Staged store: the wave writes its accumulators (as TC) into its own LDS area, rows padded by 16
 // bytes (the 16 rows x 4 column groups of one write land on distinct banks), then copies them out
 // in 16-byte row chunks, so every global store covers whole row segments.  Rows are processed in
-// passes of RPP (all WM rows for 1- and 2-byte outputs).  Requires a contiguous row (sc_n == 1)
-// with 16-byte aligned row starts at the tile's column origin.
+// passes of RPP (all WM rows for 1- and 2-byte outputs).  Requires contiguous rows of C; `aligned`:
+// every row starts 16-byte aligned at the tile's column origin.
 // Rows per staging pass: the largest multiple of 16 that divides WM (a pass takes whole 16-row
 // fragment blocks) and whose padded rows fit in the wave's staging bytes; 16 when none does, which
 // the callers' static_asserts then reject.  (Halving WM instead would give 24 rows for WM = 48.)
@@ -331,7 +333,7 @@ struct NoTransform {
 
 template <typename TC, class C, typename Acc, int WAVE_BYTES = kEpiWaveBytes, class F = NoTransform>
 __device__ inline void write_tile_staged(const Acc (&acc)[C::FM][C::FN], char* lds_wave, char* Cb, int lane, int mrow0,
-                                         int ncol0, const GemmDesc& d, const F& f = F()) {
+                                         int ncol0, const GemmDesc& d, bool aligned, const F& f = F()) {
     constexpr int ROWB = C::WN * (int)sizeof(TC);            // bytes per output row of the wave tile
     constexpr int PITCH = ROWB + 16;
     constexpr int RPP = staged_rows<C::WM, PITCH, WAVE_BYTES>(); // rows per pass
@@ -365,7 +367,8 @@ __device__ inline void write_tile_staged(const Acc (&acc)[C::FM][C::FN], char* l
             const u32x4 v = *reinterpret_cast<const u32x4*>(lds_wave + r * PITCH + c * 16);
             TC* dst = reinterpret_cast<TC*>(Cb) + (int64_t)row * d.sc_m + col;
             if (col + 16 / (int)sizeof(TC) <= d.N) {
-                if constexpr (ROWB % 128 == 0) store_stream16(dst, v); // whole lines per row
+                if (!aligned) __builtin_memcpy(dst, &v, 16);
+                else if constexpr (ROWB % 128 == 0) store_stream16(dst, v); // whole lines per row
                 else *reinterpret_cast<u32x4*>(dst) = v;
             } else {
                 const TC* e = reinterpret_cast<const TC*>(&v);
@@ -386,10 +389,10 @@ __device__ inline void write_tile_staged(const Acc (&acc)[C::FM][C::FN], char* l
 // in its LDS area (rows padded by 16 bytes), then each lane takes 4 consecutive columns of a row,
 // adds their bias values, applies the activation and stores them rounded once to TC.  The
 // accumulators are dead before the bias is read, so the epilogue adds no register pressure to the
-// k-loop.  Requires row-contiguous C (sc_n == 1); vec_ok: rows aligned for 4-element stores.
+// k-loop.  Requires row-contiguous C; aligned: rows 16-byte aligned.
 template <typename TC, class C, int WAVE_BYTES = kEpiWaveBytes>
 __device__ inline void write_tile_staged_epi(const f32x4 (&acc)[C::FM][C::FN], char* lds_wave, char* Cb, int lane,
-                                             int mrow0, int ncol0, const GemmDesc& d, int b, bool vec_ok) {
+                                             int mrow0, int ncol0, const GemmDesc& d, int b, bool aligned) {
     constexpr int ROWB = C::WN * 4;
     constexpr int PITCH = ROWB + 16;
     constexpr int RPP = staged_rows<C::WM, PITCH, WAVE_BYTES>();
@@ -449,11 +452,12 @@ __device__ inline void write_tile_staged_epi(const f32x4 (&acc)[C::FM][C::FN], c
             }
             if (row >= d.M) continue;
             TC* dst = reinterpret_cast<TC*>(Cb) + (int64_t)row * d.sc_m + col;
-            if (vec_ok && col + 4 <= d.N) {
+            if (col + 4 <= d.N) {
                 out4 o;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) o[q] = cvt_out<TC>(v[q]);
-                if constexpr (C::WN * sizeof(TC) % 128 != 0) *reinterpret_cast<out4*>(dst) = o; // part lines
+                if (!aligned) __builtin_memcpy(dst, &o, sizeof(o));
+                else if constexpr (C::WN * sizeof(TC) % 128 != 0) *reinterpret_cast<out4*>(dst) = o; // part lines
                 else if constexpr (sizeof(out4) == 16) store_stream16(dst, __builtin_bit_cast(u32x4, o));
                 else store_stream8(dst, __builtin_bit_cast(uint2, o));
             } else {
@@ -645,39 +649,39 @@ __device__ inline void mfma_tile_store(const GemmDesc& d, char* smem, int b, int
     char* Cb = static_cast<char*>(d.C) + (int64_t)b * d.sc_b * csz;
     const int row0 = m0 + wm * C::WM + (lane & 15);
     const int col0 = n0 + wn * C::WN + (lane >> 4) * 4;
-    const bool vec_ok = c_vec != 0;
+    const bool aligned = c_vec == 2;
     if constexpr (FUSED && !__is_same(Acc, i32x4)) {
         // Fused epilogue: fp32 staging, bias and activation after the accumulators are dead.
         lds_barrier();
         char* lw = smem + wave * kEpiWaveBytes;
         const int mrow0 = m0 + wm * C::WM, ncol0 = n0 + wn * C::WN;
-        if (d.dtype_c == TV_BFLOAT16) write_tile_staged_epi<__bf16, C>(acc, lw, Cb, lane, mrow0, ncol0, d, b, vec_ok);
-        else if (d.dtype_c == TV_FLOAT16) write_tile_staged_epi<_Float16, C>(acc, lw, Cb, lane, mrow0, ncol0, d, b, vec_ok);
-        else write_tile_staged_epi<float, C>(acc, lw, Cb, lane, mrow0, ncol0, d, b, vec_ok);
+        if (d.dtype_c == TV_BFLOAT16) write_tile_staged_epi<__bf16, C>(acc, lw, Cb, lane, mrow0, ncol0, d, b, aligned);
+        else if (d.dtype_c == TV_FLOAT16) write_tile_staged_epi<_Float16, C>(acc, lw, Cb, lane, mrow0, ncol0, d, b, aligned);
+        else write_tile_staged_epi<float, C>(acc, lw, Cb, lane, mrow0, ncol0, d, b, aligned);
         return;
     }
-    if (c_vec == 2) {
+    if (c_vec != 0) {
         // All waves are done with the k-loop's LDS stages before any wave reuses them.
         lds_barrier();
         char* lw = smem + wave * kEpiWaveBytes;
         const int mrow0 = m0 + wm * C::WM, ncol0 = n0 + wn * C::WN;
         if constexpr (__is_same(Acc, i32x4)) {
-            if (d.dtype_c == TV_INT8) write_tile_staged<int8_t, C>(acc, lw, Cb, lane, mrow0, ncol0, d);
-            else write_tile_staged<int32_t, C>(acc, lw, Cb, lane, mrow0, ncol0, d);
+            if (d.dtype_c == TV_INT8) write_tile_staged<int8_t, C>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
+            else write_tile_staged<int32_t, C>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
         } else {
-            if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C>(acc, lw, Cb, lane, mrow0, ncol0, d);
-            else if (d.dtype_c == TV_FLOAT16) write_tile_staged<_Float16, C>(acc, lw, Cb, lane, mrow0, ncol0, d);
-            else write_tile_staged<float, C>(acc, lw, Cb, lane, mrow0, ncol0, d);
+            if (d.dtype_c == TV_BFLOAT16) write_tile_staged<__bf16, C>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
+            else if (d.dtype_c == TV_FLOAT16) write_tile_staged<_Float16, C>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
+            else write_tile_staged<float, C>(acc, lw, Cb, lane, mrow0, ncol0, d, aligned);
         }
         return;
     }
     if constexpr (__is_same(Acc, i32x4)) {
-        if (d.dtype_c == TV_INT8) write_tile<int8_t, C>(acc, Cb, row0, col0, vec_ok, d);
-        else write_tile<int32_t, C>(acc, Cb, row0, col0, vec_ok, d);
+        if (d.dtype_c == TV_INT8) write_tile<int8_t, C>(acc, Cb, row0, col0, d);
+        else write_tile<int32_t, C>(acc, Cb, row0, col0, d);
     } else {
-        if (d.dtype_c == TV_BFLOAT16) write_tile<__bf16, C>(acc, Cb, row0, col0, vec_ok, d);
-        else if (d.dtype_c == TV_FLOAT16) write_tile<_Float16, C>(acc, Cb, row0, col0, vec_ok, d);
-        else write_tile<float, C>(acc, Cb, row0, col0, vec_ok, d);
+        if (d.dtype_c == TV_BFLOAT16) write_tile<__bf16, C>(acc, Cb, row0, col0, d);
+        else if (d.dtype_c == TV_FLOAT16) write_tile<_Float16, C>(acc, Cb, row0, col0, d);
+        else write_tile<float, C>(acc, Cb, row0, col0, d);
     }
 }
 
@@ -905,16 +909,8 @@ static int run_cfg(const GemmDesc& d, hipStream_t stream, int group_m, bool may_
     const int64_t nwg = (int64_t)tiles_m * tiles_n * d.batch;
     if (nwg <= 0) return 0;
     if (nwg > 0x7FFFFFFF) return TV_E_SHAPE;
-    const size_t csz = dtype_size(d.dtype_c);
-    // c_vec = 1: 4-element vector stores along rows of C (aligned to 4 elements);
-    // c_vec = 2: LDS-staged 16-byte row chunks (rows 16-byte aligned at every tile origin).
-    int c_vec = d.sc_n == 1 && d.sc_m % 4 == 0 && (d.batch <= 1 || d.sc_b % 4 == 0) &&
-                (reinterpret_cast<uintptr_t>(d.C) % (4 * csz)) == 0;
-    const int64_t v16 = 16 / (int64_t)csz;
-    if (c_vec && d.sc_m % v16 == 0 && (d.batch <= 1 || d.sc_b % v16 == 0) &&
-        (reinterpret_cast<uintptr_t>(d.C) % 16) == 0 && (C::WN * (int64_t)csz) % 16 == 0)
-        c_vec = 2;
-    // The fused epilogue runs in the staged store only (16-byte aligned rows of C).
+    const int c_vec = c_store_mode(d);
+    // The fused epilogue runs in the staged store only.
     const bool epi = d.bias != nullptr || d.act != TV_ACT_NONE;
     if (epi && d.sc_n != 1) return TV_E_UNSUPPORTED; // the fused store writes rows of C
     if constexpr (__is_same(typename C::T, float))

@@ -292,14 +292,6 @@ static bool ms_rotation(const GemmDesc& d, int es, int am, int64_t tiles_m, int6
     return am == LOAD_KCONTIG && (int64_t)d.K * d.N * es <= (int64_t)2 << 20 && tiles_m >= 4 * tiles_n;
 }
 
-// Whole 16-byte rows of C (2), 4-element vectors (1) or neither (0).
-template <class C> static int c_vec_of(const GemmDesc& d) {
-    const int64_t csz = (int64_t)dtype_size(d.dtype_c), v16 = 16 / csz;
-    const bool v4 = d.sc_n == 1 && d.sc_m % 4 == 0 && (d.batch <= 1 || d.sc_b % 4 == 0) &&
-                    (reinterpret_cast<uintptr_t>(d.C) % (4 * csz)) == 0;
-    return v4 && d.sc_m % v16 == 0 && (d.batch <= 1 || d.sc_b % v16 == 0) && aligned16(d.C) && (C::WN * csz) % 16 == 0 ? 2 : v4;
-}
-
 template <class C, int NST>
 static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan) {
     constexpr int kGroupM = 8;
@@ -324,7 +316,7 @@ static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan)
             ms.iters = nt * ms.nk;
         }
     }
-    const int c_vec = c_vec_of<C>(d);
+    const int c_vec = c_store_mode(d);
     if constexpr (!__is_same(typename C::T, int8_t))
         if (epi) {
             hipLaunchKernelGGL((gemm_ms_kernel<C, NST, true>), dim3((unsigned)G), dim3(C::THREADS), 0, stream, d, (int)tiles_m,

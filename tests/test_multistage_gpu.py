@@ -101,3 +101,20 @@ def test_fused_relu_bias_exact(hip, dt, shape):
                                        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
     torch.cuda.synchronize()
     np.testing.assert_array_equal(to_storage(c), want)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=["fp32", "bf16", "fp16", "int8"])
+@pytest.mark.parametrize("shape", [(40, 67, 64), (130, 257, 192), (520, 1031, 256), (2064, 1029, 128), (4096, 2047, 64)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_unaligned_rows_of_c_exact(hip, dt, shape):
+    """C rows at any alignment (odd N; a start inside wider rows): every element stored, none beside."""
+    M, N, K = shape
+    x, y = _ints(M, (M, K)), _ints(N, (K, N))
+    want = _enc(np.matmul(x.astype(np.float64), y.astype(np.float64)), dt)
+    tx, ty = _dev(x, dt, False), _dev(y, dt, True)
+    for pad, off in ((0, 0), (3, 1), (16, 5)):
+        wide = torch.full((M, N + pad), 77, dtype=tx.dtype, device="cuda")
+        hip.gemm(tx, ty, out=wide[:, off:off + N])
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(to_storage(wide[:, off:off + N].contiguous()), want)
+        assert bool((wide[:, :off] == 77).all()) and bool((wide[:, off + N:] == 77).all())
