@@ -9,6 +9,7 @@ result type instead (src/backend/cpu/mul.cpp:110-112).
 from __future__ import annotations
 
 import ctypes
+import struct
 
 import torch
 
@@ -109,39 +110,67 @@ def make_args(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> TvGemmArgs:
     return args
 
 
-def _out(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None, out_dtype: int | None) -> torch.Tensor:
-    _check_shapes(a, b)
-    dt = out_dtype if out_dtype is not None else compute_type(torch_to_tv(a.dtype), torch_to_tv(b.dtype))
-    shape = (a.shape[0], a.shape[1], b.shape[-1]) if a.dim() == 3 else (a.shape[0], b.shape[-1])
-    if out is None:
-        out = torch.empty(shape, dtype=tv_to_torch(dt), device=a.device)
-    elif tuple(out.shape) != shape or torch_to_tv(out.dtype) != dt:
-        raise RuntimeError(f"out has shape {tuple(out.shape)}/{out.dtype}, expected {shape}/{tv_to_torch(dt)}")
-    return out
+# tv_gemm_args as bytes, in native layout (the fields of make_args in order).
+_pack_args = struct.Struct("4i 4q P3q P3q P3q").pack
+assert struct.calcsize("4i 4q P3q P3q P3q") == ctypes.sizeof(TvGemmArgs)
+_entries: dict[str, object] = {}  # entry point -> ctypes function that takes the packed bytes
+
+
+def _entry(name: str):
+    fn = _entries.get(name)
+    if fn is None:
+        fn = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_char_p, ctypes.c_void_p)((name, lib()))
+        _entries[name] = fn
+    return fn
+
+
+def _current_stream() -> int:
+    # The handle of torch.cuda.current_stream(), without building the Stream object (2.8 us of a 10.5 us call).
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _stream(stream) -> int:
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+        return _current_stream()
     return stream if isinstance(stream, int) else stream.cuda_stream
+
+
+def _run(name: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None, out_dtype: int | None, stream) -> torch.Tensor:
+    """Checks, output and descriptor of one call.  A small product is bound by this host code, so it reads
+    each tensor attribute once and packs the descriptor in one step: 10.5 -> 7.0 us a call."""
+    sa, sb = a.shape, b.shape
+    if a.device != b.device or not (len(sa) == len(sb) or (len(sa) == 3 and len(sb) == 2)) or \
+            not (len(sa) == 2 or (len(sa) == 3 and (len(sb) == 2 or sa[0] == sb[0]))) or sa[-1] != sb[-2]:
+        _check_shapes(a, b)  # raises the message that applies
+    da, db = torch_to_tv(a.dtype), torch_to_tv(b.dtype)
+    dc = out_dtype if out_dtype is not None else compute_type(da, db)
+    batched = len(sa) == 3
+    m, k, n = sa[-2], sa[-1], sb[-1]
+    shape = (sa[0], m, n) if batched else (m, n)
+    if out is None:
+        out = a.new_empty(shape, dtype=_TV2T[dc])
+    elif tuple(out.shape) != shape or torch_to_tv(out.dtype) != dc:
+        raise RuntimeError(f"out has shape {tuple(out.shape)}/{out.dtype}, expected {shape}/{tv_to_torch(dc)}")
+    if batched:
+        args = _pack_args(da, db, dc, 0, sa[0], m, n, k, a.data_ptr(), *a.stride(), b.data_ptr(),
+                          *(b.stride() if len(sb) == 3 else (0, *b.stride())), out.data_ptr(), *out.stride())
+    else:
+        args = _pack_args(da, db, dc, 0, 1, m, n, k, a.data_ptr(), 0, *a.stride(), b.data_ptr(), 0, *b.stride(),
+                          out.data_ptr(), 0, *out.stride())
+    check(_entry(name)(args, _current_stream() if stream is None else _stream(stream)))
+    return out
 
 
 def gemm(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None, out_dtype: int | None = None,
          stream=None) -> torch.Tensor:
     """C = A @ B on the HIP kernels (asynchronous on ``stream``, default torch's current stream)."""
-    out = _out(a, b, out, out_dtype)
-    args = make_args(a, b, out)
-    check(lib().tv_hip_gemm(ctypes.byref(args), ctypes.c_void_p(_stream(stream))))
-    return out
+    return _run("tv_hip_gemm", a, b, out, out_dtype, stream)
 
 
 def gemv(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None, out_dtype: int | None = None,
          stream=None) -> torch.Tensor:
     """Skinny-M (M <= 8) path; raises TensorviaHipError(TV_E_UNSUPPORTED) if it does not serve the call."""
-    out = _out(a, b, out, out_dtype)
-    args = make_args(a, b, out)
-    check(lib().tv_hip_gemv(ctypes.byref(args), ctypes.c_void_p(_stream(stream))))
-    return out
+    return _run("tv_hip_gemv", a, b, out, out_dtype, stream)
 
 
 def matmul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
