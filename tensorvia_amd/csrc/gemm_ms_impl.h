@@ -73,23 +73,28 @@ __device__ __attribute__((always_inline)) inline void ms_tile_kloop(const GemmDe
     la.xinit(LA0, lane, wm * C::WM);
     lb.xinit(LB0, lane, wn * C::WN);
 
-    auto issue = [&](int kt, int st) {
-        if (kt < kt1) { // past the range: zeros, from the loaders' K
+    auto k_of = [&](int kt) { // past the range: zeros, from the loaders' K
+        if (kt < kt1) {
             kt += rot;
             kt = kt < kt1 ? kt : kt - (kt1 - kt0);
         }
-        la.issue(L + st * LA::BYTES, wave, kt * C::BK);
-        lb.issue(L + NST * LA::BYTES + st * LB::BYTES, wave, kt * C::BK);
+        return kt * C::BK;
+    };
+    auto issue = [&](int kt, int st) {
+        la.issue(L + st * LA::BYTES, wave, k_of(kt));
+        lb.issue(L + NST * LA::BYTES + st * LB::BYTES, wave, k_of(kt));
     };
     // A fragments: one set, each reloaded with the next k-group's right after its row of MFMAs; B
     // fragments: one set per k-group.
     u32x4 fa[C::FM], fb[2][C::FN];
-    // MFMAs of one k-group (B set `cur`), reading k-group kg of the k-tile at xa / xb into the other set.
-    auto kgroup = [&](int cur, unsigned xa, unsigned xb, int kg) {
+    // MFMAs of one k-group (B set `cur`), reading k-group kg of the k-tile at xa / xb into the other set;
+    // after(i) runs behind row i's MFMAs.
+    auto kgroup = [&](int cur, unsigned xa, unsigned xb, int kg, const auto& after) {
 #pragma unroll
         for (int i = 0; i < C::FM; ++i) {
 #pragma unroll
             for (int j = 0; j < C::FN; ++j) Op::run(fb[cur][j], fa[i], acc[i][j]);
+            after(i);
             fa[i] = LA::frag_from(xa, 0, kg, i);
 #pragma unroll
             for (int j = i * C::FN / C::FM; j < (i + 1) * C::FN / C::FM; ++j) fb[cur ^ 1][j] = LB::frag_from(xb, 0, kg, j);
@@ -113,12 +118,34 @@ __device__ __attribute__((always_inline)) inline void ms_tile_kloop(const GemmDe
     for (int i = 0; i < C::FM; ++i) fa[i] = LA::frag_from(la.xf, 0, 0, i);
     int st = 0;
     auto ktile = [&](int kt) {
-        wait_vmcnt<(NST - 3) * NDMA>();
-        dma_barrier();
-        issue(kt + NST - 1, st == 0 ? NST - 1 : st - 1);
-        kgroup(0, la.xf + (unsigned)(st * LA::BYTES), lb.xf + (unsigned)(st * LB::BYTES), 1);
+        const int fs = st == 0 ? NST - 1 : st - 1; // the stage freed last step
+        const unsigned xa = la.xf + (unsigned)(st * LA::BYTES), xb = lb.xf + (unsigned)(st * LB::BYTES);
+        // The loads of k-tile t + NST - 1.  On the small 16-bit and int8 tiles they go out between the
+        // rows of MFMAs, beside which their issue (about 40 cycles each) runs: bf16
+        // [128,4096]@Wt[4096,4096] on 64x64 tiles 20.4 -> 18.8 us.  On the large tiles, whose second wave
+        // per SIMD covers it, and in fp32 all at once (128x128: bf16 [1024,4096]@[4096,4096] 41.1 us, 42.8
+        // between the rows; fp32 [1024]^3 23.5, 26.2).
+        if constexpr (ES <= 2 && C::FM * C::FN <= 4) {
+            const int k2 = k_of(kt + NST - 1);
+            const __amdgpu_buffer_rsrc_t ra = la.rsrc(k2), rb = lb.rsrc(k2);
+            const unsigned sa = LA0 + (unsigned)(fs * LA::BYTES), sb = LB0 + (unsigned)(fs * LB::BYTES);
+            wait_vmcnt<(NST - 3) * NDMA>();
+            dma_barrier();
+            kgroup(0, xa, xb, 1, [&](int i) {
+#pragma unroll
+                for (int u = i * NDMA / C::FM; u < (i + 1) * NDMA / C::FM; ++u) {
+                    if (u < LA::PER_WAVE) la.issue_one(u, ra, sa, wave, k2);
+                    else lb.issue_one(u - LA::PER_WAVE, rb, sb, wave, k2);
+                }
+            });
+        } else {
+            wait_vmcnt<(NST - 3) * NDMA>();
+            dma_barrier();
+            issue(kt + NST - 1, fs);
+            kgroup(0, xa, xb, 1, [](int) {});
+        }
         st = st + 1 == NST ? 0 : st + 1;
-        kgroup(1, la.xf + (unsigned)(st * LA::BYTES), lb.xf + (unsigned)(st * LB::BYTES), 0);
+        kgroup(1, la.xf + (unsigned)(st * LA::BYTES), lb.xf + (unsigned)(st * LB::BYTES), 0, [](int) {});
     };
     // fp32 results in chunks of kChunk k-tiles, each summed by itself and then added: rounding grows
     // with the chunk's length and the chunk count, not with K (fp32 [1001,777]@[777,1003]: 2.6e-7
@@ -274,7 +301,10 @@ static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool
             if (best.tile < 0 || us < best.us) best = MsPlan{i, wgs, split, us};
         };
         const int64_t full = nt / slots, rest = nt % slots;
-        offer(nt, false, nk * (full * step(slots) + (rest ? step(rest) : 0)), t.round * (double)(full + (rest != 0) - 1));
+        // A CU's second and third workgroup start beside the first, not for nothing (fp16
+        // [13][128,512]@[512,928] on 390 tiles of 64x64 11.2 us, 9.4 on 128x128).
+        const double start = t.s0 < 0 || t.occ == 1 || nt <= cus ? 0.0 : 1.5 * (double)((nt < slots ? (nt + cus - 1) / cus : t.occ) - 1);
+        offer(nt, false, nk * (full * step(slots) + (rest ? step(rest) : 0)), start + t.round * (double)(full + (rest != 0) - 1));
         if (!may_split || t.s0 < 0 || nt > 0x3FFFFFFF / (nk > 0 ? nk : 1)) continue;
         for (int s = 2; s <= 64 && nt * s <= slots && nk >= 2 * s; s += s < 8 ? 1 : s / 4)
             offer(nt * s, true, (double)nk / s * step(nt * s), t.s0 + t.s1 * s);
@@ -336,9 +366,9 @@ static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan)
 // two workgroups per CU, which start faster (bf16 [8][512,96]@Kt[96,512] 5.0 us against 6.2 here), and
 // 256x256 tiles (bf16 [4096]^3 98 us).
 enum { MS_32x64, MS_64x64, MS_64x128, MS_128x128, MS_256x128, MS_DMA_128, MS_DMA_256, MS_TILES };
-constexpr MsTile kMsTiles[MS_TILES] = {{32, 64, 3, 3.5, 2.0, 0.25, 0.43, 3.0, 0.25},  {64, 64, 2, 4.5, 2.6, 0.25, 0.43, 3.0, 0.25},
-                                       {64, 128, 1, 4.0, 3.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.58, 0.58, 5.0, 0.6},
-                                       {256, 128, 1, 6.5, 5.5, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.67, 1.03, -1, 0},
+constexpr MsTile kMsTiles[MS_TILES] = {{32, 64, 3, 3.5, 2.0, 0.25, 0.43, 3.0, 0.25},  {64, 64, 2, 4.8, 2.6, 0.25, 0.43, 3.0, 0.25},
+                                       {64, 128, 1, 5.0, 3.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.58, 0.58, 5.0, 0.6},
+                                       {256, 128, 1, 6.5, 5.5, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.67, 0.95, -1, 0},
                                        {256, 256, 1, 9.0, 7.0, 1.3, 1.3, -1, 0}};
 
 // Runs d on the cheapest tile; 1 if that is the 256x256 one.  am / bm: the operands' (vector) load modes.
@@ -348,13 +378,16 @@ static int run_modes_ms(const GemmDesc& d, hipStream_t stream, int group_m, int 
     const int nk = (d.K + 128 / (int)sizeof(T) - 1) / (128 / (int)sizeof(T));
     // Layouts: 32 rows K-contiguous only; 64 rows M/N-contiguous at 16 bits only (DmaOperand).
     const bool r64a = am == LOAD_KCONTIG || !kI8, r64b = bm == LOAD_KCONTIG || !kI8;
-    // Tall calls whose tiles stream A in rows of k, more than 64 columns wide and enough of them for
-    // 256x128 tiles: that tile, rotated, whatever the prices (bf16 [65536,2048]@[2048,128] 57 us, 62 on
+    // Tall calls whose tiles stream A in rows of k with a pitch of whole 2 KB, more than 64 columns wide
+    // and enough of them for 256x128 tiles: that tile, rotated, whatever the prices (bf16 [65536,2048]@[2048,128] 57 us, 62 on
     // 128x128 tiles; 74 unrotated, on the two-stage 128x128 tiles as well).
     const int64_t tall_m = ((int64_t)d.M + 255) / 256 * d.batch, tall_n = (d.N + 127) / 128;
-    const bool tall = d.N > 64 && nk >= 8 && tall_m * tall_n * 4 >= 3 * (int64_t)device_cus() &&
+    const bool tall = d.N > 64 && nk >= 8 && d.sa_m * (int64_t)sizeof(T) % 2048 == 0 && tall_m * tall_n * 4 >= 3 * (int64_t)device_cus() &&
                       ms_rotation(d, (int)sizeof(T), am, tall_m, tall_n);
-    const bool ok[MS_TILES] = {am == LOAD_KCONTIG && r64b, r64a && r64b, kI8 && am == LOAD_KCONTIG && !r64b, true, true, true, true};
+    // 32x64 tiles up to one per CU: more of them read B from L2 too often (fp16 [3][128,448]@[448,2744],
+    // 516 tiles, 12.7 us; 9.2 on 64x64 or 128x128).
+    const bool few32 = ((int64_t)d.M + 31) / 32 * (((int64_t)d.N + 63) / 64) * d.batch <= device_cus();
+    const bool ok[MS_TILES] = {am == LOAD_KCONTIG && r64b && few32, r64a && r64b, kI8 && am == LOAD_KCONTIG && !r64b, true, true, true, true};
     MsPlan plan = ms_plan(d, nk, kMsTiles, ok, MS_TILES, may_alloc);
     if (tall) plan = MsPlan{MS_256x128, 0, false, 0};
     if (plan.tile == MS_DMA_256) return 1;
