@@ -121,6 +121,16 @@ int run_gemm(const tv_gemm_args* args, const tvk::GemmDesc& d0, hipStream_t s, c
     if (d0.batch == 0 || d0.M == 0 || d0.N == 0) return TV_OK;
     if (mfma_pair(args) && d0.K == 0) return tvk::launch_gemm_k0(d0, s);
     tvk::GemmDesc d = d0;
+    // The smallest products: the GEMV where it takes the layout (M <= 8), else one 16 x 16 block per
+    // workgroup, before any operand is copied.
+    if (mfma_pair(args) && d.M <= 128 && d.N <= 128 && d.K <= 128) {
+        if (d.M <= 8) {
+            const int rc = tvk::launch_gemv(d, s, fixed);
+            if (rc != TV_E_UNSUPPORTED && rc != TV_E_NOMEM) return rc;
+        }
+        const int rc = tvk::launch_gemm_tiny(d, s);
+        if (rc != TV_E_UNSUPPORTED) return rc;
+    }
     if (mfma_pair(args) && fixed == nullptr) { // misaligned operands into padded rows (workspace)
         const int rc = tvk::pad_gemm_operands(d, s);
         if (rc) return rc;

@@ -118,3 +118,26 @@ def test_unaligned_rows_of_c_exact(hip, dt, shape):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(to_storage(wide[:, off:off + N].contiguous()), want)
         assert bool((wide[:, :off] == 77).all()) and bool((wide[:, off + N:] == 77).all())
+
+
+TINY = [(1, 1, 1), (9, 15, 1), (16, 16, 128), (17, 33, 129), (31, 128, 33), (128, 128, 128), (129, 16, 64), (9, 1, 127)]
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=["fp32", "bf16", "fp16", "int8"])
+@pytest.mark.parametrize("shape", TINY, ids=lambda s: "x".join(map(str, s)))
+def test_smallest_products_exact(hip, dt, shape):
+    """The 16 x 16-block kernel of the smallest products, its edges and one past its limits: row-major,
+    transposed and column-stepped operands, batches, a column-strided C."""
+    M, N, K = shape
+    x, y = _ints(M + K, (3, M, K)), _ints(N + K, (3, K, N))
+    want = _enc(np.matmul(x.astype(np.float64), y.astype(np.float64)), dt)
+    for at in (False, True):
+        for bt in (False, True):
+            np.testing.assert_array_equal(to_storage(hip.gemm(_dev(x, dt, at), _dev(y, dt, bt))), want)
+    wide = np.zeros((3, M, 2 * K), x.dtype)
+    wide[..., ::2] = x
+    np.testing.assert_array_equal(to_storage(hip.gemm(_dev(wide, dt, False)[..., ::2], _dev(y, dt, False))), want)
+    c = torch.zeros((3, N, M), dtype=_dev(x[:1], dt, False).dtype, device="cuda").transpose(1, 2)
+    hip.gemm(_dev(x, dt, False), _dev(y, dt, False), out=c)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(to_storage(c.contiguous()), want)
