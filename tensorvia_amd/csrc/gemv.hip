@@ -718,6 +718,11 @@ static int get_workspace(hipStream_t stream, size_t need, void** out, int kind) 
     GemvWorkspace& w = g_ws[{dev, stream, kind}];
     const bool fail = alloc_failure_armed(); // test hook: this request fails as an allocation would
     if (w.bytes < need || fail) {
+        // A stream under capture can neither allocate nor be synchronised: the call takes its path
+        // without the buffer, as when memory is exhausted.
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
+        if (cap != hipStreamCaptureStatusNone) return TV_E_NOMEM;
         if (w.base && !fail) {
             // The old buffer may still be in use by queued work of this stream.
             e = hipStreamSynchronize(stream);

@@ -141,3 +141,25 @@ def test_smallest_products_exact(hip, dt, shape):
     hip.gemm(_dev(x, dt, False), _dev(y, dt, False), out=c)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(to_storage(c.contiguous()), want)
+
+
+@pytest.mark.parametrize("dt", [FLOAT32, BFLOAT16, INT8], ids=["fp32", "bf16", "int8"])
+@pytest.mark.parametrize("shape", [(64, 64, 8192), (48, 1216, 3712), (65, 77, 2049)], ids=lambda s: "x".join(map(str, s)))
+def test_cold_capture_exact(hip, dt, shape):
+    """A call that wants a workspace, captured on a stream that has none yet: the captured call runs
+    without it, and every replay gives the exact result, eager calls of the same shape between."""
+    M, N, K = shape
+    x, y = _ints(M, (M, K)), _ints(N, (K, N))
+    want = _enc(np.matmul(x.astype(np.float64), y.astype(np.float64)), dt)
+    tx, ty = _dev(x, dt, False), _dev(y, dt, True)
+    out = torch.zeros((M, N), dtype=tx.dtype, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        hip.gemm(tx, ty, out=out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(to_storage(out), want)
+        np.testing.assert_array_equal(to_storage(hip.gemm(tx, ty)), want)
