@@ -48,8 +48,9 @@
  *   - bf16/fp16 inputs: fp32 accumulation, output bf16/fp16 (GPU-backend convention) or FLOAT32
  *     (the CPU backend's widened result);
  *   - fp32: fp32 accumulation on the fp32 matrix cores;
+ *   - fp64: fp64 accumulation on the fp64 matrix cores, in the reference CPU order;
  *   - any other dtype pair: exact restatement of the reference CPU accumulation rules on a
- *     SIMT kernel (slow path, provided for completeness).
+ *     tiled SIMT kernel.
  *
  * Calls are asynchronous on `hip_stream` (a hipStream_t, NULL = default stream).  The caller
  * keeps A, B and C alive until the stream has executed the work.  The split-K schedules keep their

@@ -186,8 +186,8 @@ inline int pick_mode(const void* p, int64_t R, int64_t K, int64_t s_r, int64_t s
 }
 
 // Launchers (return hipError_t, or a negative TV_E_* code).
-// may_alloc = false: no launch path that needs a grown workspace (the stream-K schedule of the fp32
-// kernel); the plain data-parallel kernels serve the call.
+// may_alloc = false: no launch path that needs a grown workspace (tiles split over K); the plain
+// data-parallel kernels serve the call.
 int launch_gemm_mfma(const GemmDesc& d, hipStream_t stream, bool may_alloc = true);
 // Copies operands that are contiguous along one dimension but not in whole 16-byte rows into
 // zero-padded rows in the per-stream workspace (calls of at least 2^20 multiply-adds or K >= 256) and points d
