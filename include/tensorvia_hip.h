@@ -147,7 +147,7 @@ int tv_hip_gemm_ex(const tv_gemm_args* args, const tv_epilogue* ep, void* hip_st
  * forbid hipMalloc).  Same arguments and routing as tv_hip_gemm.  The split-K partials of the
  * M <= 8 GEMV kernels come from a static device array of 4 MiB of partial slots plus 16,384 arrival
  * counters per GPU, held until the process ends, instead of tv_hip_gemm's workspace.  GEMMs
- * (M > 8) that tv_hip_gemm splits with its stream-K schedule, whose partial tiles need a
+ * that tv_hip_gemm splits over K, whose partial tiles need a
  * workspace, run unsplit here, so their fp32 and 16-bit results can differ from tv_hip_gemm's in
  * the last bits (summation order).  So can float calls with an operand whose rows are not whole
  * 16-byte chunks (e.g. bf16 W[4096,129]): tv_hip_gemm copies such an operand into padded rows (a
