@@ -58,8 +58,11 @@
  * 16-byte chunks, in a workspace per (device, stream): calls on one stream are ordered by that
  * stream, and calls on different streams use different workspaces, so concurrent streams are safe.
  * Growing a stream's workspace synchronises that stream once.  When the workspace cannot be
- * allocated (device memory exhausted), the call runs on kernels that need none (the unsplit GEMM,
- * the element-gather loader), more slowly, and still returns 0.
+ * allocated (device memory exhausted, or the stream is under capture and no earlier eager call made
+ * it large enough), the call runs on kernels that need none (the unsplit GEMM, the element-gather
+ * loader, the GEMM in place of the split-K GEMV), more slowly, and still returns 0.  A captured graph
+ * keeps the buffers it recorded: they are neither freed nor used by eager calls afterwards; graphs
+ * captured on one stream share them and must not run at the same time.
  */
 #ifndef TENSORVIA_HIP_H
 #define TENSORVIA_HIP_H

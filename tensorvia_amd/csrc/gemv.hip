@@ -686,13 +686,18 @@ __global__ __launch_bounds__(256) void gemv_zero_kernel(int* p, int64_t n) {
 namespace tvk {
 
 // Per-(device, stream, kind) workspace.  Calls on one stream are ordered by the stream, so they
-// can share it.
-struct GemvWorkspace {
+// can share a buffer.  A captured graph keeps the address it recorded and may be replayed on any
+// stream at any time, so a buffer that a capture was given is never freed and never given to an eager
+// call again: `graph` serves the captures of the stream, `eager` everything else.
+struct Buffer {
     void* base = nullptr;
     size_t bytes = 0;
 };
+struct StreamWorkspace {
+    Buffer eager, graph;
+};
 static std::mutex g_ws_mu;
-static std::map<std::tuple<int, hipStream_t, int>, GemvWorkspace> g_ws;
+static std::map<std::tuple<int, hipStream_t, int>, StreamWorkspace> g_ws;
 
 // Test hook (tv_hip_inject_alloc_failure): while armed, each workspace request allocates, asking the
 // runtime for more memory than any device has, so it fails as it would under memory pressure (a
@@ -710,30 +715,52 @@ void inject_alloc_failure(int count) { g_alloc_fail.store(count < 0 ? 0 : count)
 // kind 1: the GEMV's split-K arrival counters (every launch leaves them at zero); kind 2: its strip
 // partial slots; kinds 3 and 4: the same for the stream-K GEMM schedule (gemm_sk_workspace); kinds
 // 5 and 6: the zero-padded copies of GEMM operands A and B (gemm_pad_workspace).
+//
+// Under capture nothing can be allocated or waited for.  A capture uses the stream's graph buffer; where
+// that is too small it takes over the eager buffer, if a warm-up made that large enough (the next eager
+// call allocates a new one, and a graph buffer it replaces stays allocated for the graphs that recorded
+// it); else the call runs without the buffer, as when memory is exhausted.  Sizes come in quarters of a
+// power of two, so the buffers that ever larger captures leave behind sum to a small multiple of the last.
 static int get_workspace(hipStream_t stream, size_t need, void** out, int kind) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusNone;
+    }
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    GemvWorkspace& w = g_ws[{dev, stream, kind}];
+    StreamWorkspace& ws = g_ws[{dev, stream, kind}];
     const bool fail = alloc_failure_armed(); // test hook: this request fails as an allocation would
+    if (cap != hipStreamCaptureStatusNone) {
+        if (fail) return TV_E_NOMEM;
+        if (ws.graph.bytes < need) {
+            if (ws.eager.bytes < need) return TV_E_NOMEM;
+            ws.graph = ws.eager;
+            ws.eager = Buffer{};
+        }
+        *out = ws.graph.base;
+        return 0;
+    }
+    Buffer& w = ws.eager;
     if (w.bytes < need || fail) {
-        // A stream under capture can neither allocate nor be synchronised: the call takes its path
-        // without the buffer, as when memory is exhausted.
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
-        if (cap != hipStreamCaptureStatusNone) return TV_E_NOMEM;
         if (w.base && !fail) {
             // The old buffer may still be in use by queued work of this stream.
             e = hipStreamSynchronize(stream);
             if (e != hipSuccess) return e;
             (void)hipFree(w.base);
-            w.base = nullptr;
-            w.bytes = 0;
+            w = Buffer{};
         }
-        const size_t sz = need < ((size_t)1 << 20) ? ((size_t)1 << 20) : need;
+        size_t sz = (size_t)1 << 20;
+        while (sz < need) sz += (size_t)1 << (61 - __builtin_clzll(sz)); // a quarter of its power of two
         void* p = nullptr;
         e = hipMalloc(&p, fail ? kImpossibleBytes : sz);
+        if (e != hipSuccess && !fail && sz > need) {
+            (void)hipGetLastError();
+            sz = need;
+            e = hipMalloc(&p, sz);
+        }
         if (e != hipSuccess) {
             // The caller may carry on without the buffer (another kernel, the gather loader): the
             // failed allocation must not stay behind as the runtime's last error, which the
@@ -741,10 +768,8 @@ static int get_workspace(hipStream_t stream, size_t need, void** out, int kind) 
             (void)hipGetLastError();
             return TV_E_NOMEM;
         }
-        w.base = p;
-        w.bytes = sz;
-        // The arrival counters must start at zero (each launch leaves them at zero again).  This
-        // workspace is not meant for stream capture: growing it synchronises the stream.
+        w = Buffer{p, sz};
+        // The arrival counters must start at zero (each launch leaves them at zero again).
         hipLaunchKernelGGL(gemv_zero_kernel, dim3(256), dim3(256), 0, stream, static_cast<int*>(w.base),
                            (int64_t)(sz / sizeof(int)));
         e = hipGetLastError();

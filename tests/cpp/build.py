@@ -22,6 +22,16 @@ def build(verbose: bool = False) -> None:
                  f"-Wl,-rpath,{be.PKG}", "-Wl,-rpath,$ORIGIN/../../../tensorvia_amd",
                  f"-Wl,-rpath,{bh.ROCM}/lib"], verbose)
         os.replace(tmp, out)
+    build_route_driver(verbose)
+
+
+def build_route_driver(verbose: bool = False) -> None:
+    """route_driver stands in for the HIP runtime: it exports its own definitions and links no ROCm library."""
+    out = BIN / "route_driver"
+    tmp = out.with_suffix(".tmp")
+    be._run([bh.CXX, "-std=c++20", "-O1", "-Wall", "-rdynamic", f"-I{be.INCLUDE}", str(HERE / "route_driver.cpp"),
+             "-o", str(tmp), "-ldl"], verbose)
+    os.replace(tmp, out)
 
 
 # Host-side AddressSanitizer + UndefinedBehaviorSanitizer build of the C++ API's CPU path: the

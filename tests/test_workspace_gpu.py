@@ -160,3 +160,55 @@ def test_workspace_users_captured_after_a_warm_up(hip):
         torch.cuda.synchronize()
         for name, want, ops, tc, args in calls:
             np.testing.assert_array_equal(to_storage(tc), want, err_msg=f"{name}: replay {rep}")
+
+
+def test_captured_graph_survives_a_larger_eager_call(hip):
+    """Graphs of workspace users, captured after a warm-up on stream s; then eager calls on s that need
+    larger buffers of each kind.  The graph's replays stay exact, on s and on another stream beside eager
+    calls of the same shapes on s (the graph's buffers are its own)."""
+    L = tv.lib()
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    shapes = [(BFLOAT16, (48, 3712), (3712, 1216), 2), (BFLOAT16, (1, 4096), (4096, 4096), 2), (BFLOAT16, (64, 700), (700, 260), 2),
+              (INT8, (48, 4096), (4096, 1216), 100)]
+    larger = [(BFLOAT16, (333, 4096), (4096, 11008), 2), (FLOAT32, (2592, 2048), (2048, 4096), 2),
+              (BFLOAT16, (8, 4096), (4096, 11008), 2), (BFLOAT16, (1000, 2047), (2047, 2049), 2)]
+
+    def calls_of(spec, seed):
+        out = []
+        for i, (dt, sa, sb, r) in enumerate(spec):
+            a, b = _int_operands(dt, sa, sb, seed + 2 * i, -r, r)
+            ta, tb = to_torch(a, dt), to_torch(b, dt)
+            tc = torch.zeros((sa[0], sb[1]), dtype=ta.dtype, device="cuda")
+            out.append((_exact(dt, a, b), (ta, tb), tc, tv.make_args(ta, tb, tc)))
+        return out
+
+    def launch(calls, stream):
+        for _, _, _, args in calls:
+            tv.check(L.tv_hip_gemm(ctypes.byref(args), ctypes.c_void_p(stream.cuda_stream)))
+
+    def check(calls, what):
+        for want, _, tc, _ in calls:
+            np.testing.assert_array_equal(to_storage(tc), want, err_msg=what)
+            tc.fill_(5)
+
+    captured, eager, big = calls_of(shapes, 1200), calls_of(shapes, 1300), calls_of(larger, 1400)
+    torch.cuda.synchronize()
+    launch(captured, s)
+    s.synchronize()
+    check(captured, "warm-up")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        launch(captured, s)
+    launch(big, s)  # larger slots, counters and padded copies
+    torch.cuda.synchronize()
+    check(big, "larger eager calls")
+    for rep in range(3):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(t):
+            g.replay()
+        for _ in range(4):
+            launch(eager, s)
+        torch.cuda.synchronize()
+        check(captured, f"replay {rep}")
+        check(eager, f"eager calls beside replay {rep}")
