@@ -43,7 +43,11 @@ bool f32_whole_rounds_256(const GemmDesc& d) {
     return tiles >= cus && tiles % cus == 0;
 }
 
-int pick_f32_tile(const GemmDesc& d, double* us) {
+// What these kernels do per us on all CUs ([2592,2048]@[2048,4096]), and the shortest time of a k-tile (32 k)
+// in a workgroup, its loads' latency: K = 4096 took 89 to 96 us on 2 to 64 workgroups of 32x128, whatever M and N.
+constexpr double kF32MacsPerUs = 64.4e6, kF32KTileUs = 0.72;
+
+int pick_f32_tile(const GemmDesc& d, bool may_split, double* us) {
     const int bm = f32_b_mode(d);
     const bool t96_ok = f32_a_mode_96(d) == LOAD_KCONTIG && (bm == LOAD_MNCONTIG || bm == LOAD_KCONTIG);
     int best = 0;
@@ -64,7 +68,13 @@ int pick_f32_tile(const GemmDesc& d, double* us) {
     // split between the workgroups (fp32 [1024]^3 37.9 us, [300,4096]@[4096,4096] 99.7 us).
     const F32Tile& t = kF32Tiles[best];
     const int64_t tiles = (int64_t)((d.M + t.bm - 1) / t.bm) * ((d.N + t.bn - 1) / t.bn) * d.batch;
-    *us = best_cost * d.K / 64.4e6 + (tiles < 512 ? 16.0 : 5.0);
+    if (may_split) {
+        *us = best_cost * d.K / kF32MacsPerUs + (tiles < 512 ? 16.0 : 5.0);
+    } else { // whole tiles: as long as the CU with the most of them
+        const int cus = device_cus();
+        const double ktile = (double)((tiles + cus - 1) / cus) * t.bm * t.bn * 32 / t.rate / (kF32MacsPerUs / 256);
+        *us = (d.K + 31) / 32 * (ktile > kF32KTileUs ? ktile : kF32KTileUs) + 5.0;
+    }
     return best;
 }
 
@@ -96,8 +106,9 @@ int run_f32_ms(const GemmDesc& d, hipStream_t stream, bool may_alloc, double oth
 
 int launch_gemm_mfma_f32(const GemmDesc& d, hipStream_t stream, bool may_alloc) {
     double us = 0;
-    const int tile = pick_f32_tile(d, &us);
+    const int tile = pick_f32_tile(d, may_alloc, &us);
     const int rc = run_f32_ms(d, stream, may_alloc, us);
+    if (rc == TV_E_NOMEM) return launch_gemm_mfma_f32(d, stream, false);
     if (rc != 1) return rc;
     switch (tile) {
         case 0:

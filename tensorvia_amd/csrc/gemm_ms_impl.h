@@ -322,6 +322,9 @@ static bool ms_rotation(const GemmDesc& d, int es, int am, int64_t tiles_m, int6
     return am == LOAD_KCONTIG && (int64_t)d.K * d.N * es <= (int64_t)2 << 20 && tiles_m >= 4 * tiles_n;
 }
 
+// TV_E_NOMEM: no room for the slots of a split plan; the caller plans again without a split (the tile
+// chosen for a split may be a poor one whole: bf16 [333,4096]@[4096,11008], 258 tiles of 128x128 that
+// fill one CU each, are two rounds of 64 k-tiles).
 template <class C, int NST>
 static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan) {
     constexpr int kGroupM = 8;
@@ -340,11 +343,9 @@ static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan)
     int64_t G = nt;
     if (plan.split) {
         const int rc = gemm_sk_workspace(stream, (size_t)nt, (size_t)2 * plan.wgs * sk_slot_bytes<C>(), &ms.cnt, &ms.slots);
-        if (rc && rc != TV_E_NOMEM) return rc;
-        if (rc == 0) { // no room for the slots: a tile per workgroup
-            G = plan.wgs;
-            ms.iters = nt * ms.nk;
-        }
+        if (rc) return rc;
+        G = plan.wgs;
+        ms.iters = nt * ms.nk;
     }
     const int c_vec = c_store_mode(d);
     if constexpr (!__is_same(typename C::T, int8_t))
@@ -371,7 +372,7 @@ constexpr MsTile kMsTiles[MS_TILES] = {{32, 64, 3, 3.5, 2.0, 0.25, 0.43, 3.0, 0.
                                        {256, 128, 1, 6.5, 5.5, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.67, 0.95, -1, 0},
                                        {256, 256, 1, 9.0, 7.0, 1.3, 1.3, -1, 0}};
 
-// Runs d on the cheapest tile; 1 if that is the 256x256 one.  am / bm: the operands' (vector) load modes.
+// Runs d on the cheapest tile; 1 if that is the 256x256 one, TV_E_NOMEM as run_ms_cfg.  am / bm: the operands' (vector) load modes.
 template <typename T>
 static int run_modes_ms(const GemmDesc& d, hipStream_t stream, int group_m, int am, int bm, bool may_alloc) {
     constexpr bool kI8 = __is_same(T, int8_t);
@@ -432,7 +433,8 @@ static int run_modes_dma(const GemmDesc& d, hipStream_t stream, int group_m, boo
     const bool epi = d.bias != nullptr || d.act != TV_ACT_NONE;
     const bool smallk = !epi && smallk_ok(d, es, 256, 256);
     if (!smallk) {
-        const int rc = run_modes_ms<T>(d, stream, group_m, am, bm, may_alloc);
+        int rc = run_modes_ms<T>(d, stream, group_m, am, bm, may_alloc);
+        if (rc == TV_E_NOMEM) rc = run_modes_ms<T>(d, stream, group_m, am, bm, false);
         if (rc != 1) return rc;
     }
 #define TV_CASE(A_, B_)                                                                         \

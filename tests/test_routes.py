@@ -1,0 +1,37 @@
+"""Which kernel, tile and grid a call gets, on the recorded runtime of tests/cpp/route_driver.cpp (no GPU,
+256 CUs)."""
+import pytest
+
+from tests.routes import call, run
+from tests.util import BFLOAT16, FLOAT16, FLOAT32, INT8
+
+SPLIT = {
+    "bf16_prompt": dict(M=333, K=4096, N=11008, dt=BFLOAT16),
+    "bf16_prompt_fused": dict(M=333, K=4096, N=11008, dt=BFLOAT16, act=2, bias=1),
+    "bf16_256x128": dict(M=130, K=8208, N=8000, dt=BFLOAT16),
+    "f16_nk": dict(M=48, K=3712, N=1216, dt=FLOAT16, bt=True),
+    "int8": dict(M=128, K=4096, N=2048, dt=INT8, bt=True),
+    "fp32": dict(M=64, K=8192, N=64, dt=FLOAT32),
+    "fp32_nk": dict(M=300, K=2048, N=320, dt=FLOAT32, bt=True),
+}
+
+
+@pytest.mark.parametrize("name", SPLIT)
+def test_without_a_workspace_the_call_is_planned_again(name):
+    """A call that splits K runs, without room for the slots (under a cold capture, or with allocations
+    failing), on the tiles that a plan without a split chooses: tv_hip_gemm_noalloc's."""
+    shape = SPLIT[name]
+    whole, cold, failed, split = run("fail 0", *([call(**shape, entry="noalloc")] if "act" not in shape else ["fail 1000", call(**shape), "fail 0"]),
+                                     "capture 1", call(**shape), "capture 0", "fail 1000", call(**shape), "fail 0", call(**shape))
+    assert split.launches[-1] != whole.launches[-1], "the call is not split"
+    for r in (cold, failed):
+        assert r.rc == 0 and r.launches[-1] == whole.launches[-1]
+
+
+@pytest.mark.parametrize("shape", [(64, 8192, 64), (300, 2048, 320), (128, 4096, 128), (256, 4096, 256)], ids=str)
+def test_fp32_few_long_tiles_without_a_workspace(shape):
+    """Unsplit, a 32-row tile of the two-stage kernel takes 22 ns per k whatever its size: the multi-stage tiles
+    are cheaper, also where the split two-stage kernel would have been."""
+    M, K, N = shape
+    for r in run(call(M, K, N, FLOAT32, entry="noalloc"), "capture 1", call(M, K, N, FLOAT32)):
+        assert r.rc == 0 and r.kernel.startswith("gemm_ms_kernel<GemmCfg<float")
