@@ -1,6 +1,8 @@
 // float instantiation of the MFMA GEMM kernels (gemm_mfma_impl.h).
 #include "gemm_ms_impl.h"
 
+#include <algorithm>
+
 namespace tvk {
 // fp32 matrix cores are 16x slower than the 16-bit ones, so a tile's wasted rows and columns cost
 // real time (a 128-row tile computes 128 rows however few are real), and few large tiles leave CUs
@@ -44,8 +46,8 @@ bool f32_whole_rounds_256(const GemmDesc& d) {
 }
 
 // What these kernels do per us on all CUs ([2592,2048]@[2048,4096]), and the shortest time of a k-tile (32 k)
-// in a workgroup, its loads' latency: K = 4096 took 89 to 96 us on 2 to 64 workgroups of 32x128, whatever M and N.
-constexpr double kF32MacsPerUs = 64.4e6, kF32KTileUs = 0.72;
+// in a workgroup, its loads' latency: K = 4096 takes 89 to 96 us on 2 to 64 workgroups of 32x128, whatever M and N.
+constexpr double kF32MacsPerUs = 64.4e6, kF32KTileUs = 0.70;
 
 int pick_f32_tile(const GemmDesc& d, bool may_split, double* us) {
     const int bm = f32_b_mode(d);
@@ -64,16 +66,22 @@ int pick_f32_tile(const GemmDesc& d, bool may_split, double* us) {
             best_cost = cost;
         }
     }
-    // The chosen tile's time: c1's rate, and what a launch costs beside it, more where few tiles are
-    // split between the workgroups (fp32 [1024]^3 37.9 us, [300,4096]@[4096,4096] 99.7 us).
+    // The chosen tile's time.
     const F32Tile& t = kF32Tiles[best];
     const int64_t tiles = (int64_t)((d.M + t.bm - 1) / t.bm) * ((d.N + t.bn - 1) / t.bn) * d.batch;
-    if (may_split) {
-        *us = best_cost * d.K / kF32MacsPerUs + (tiles < 512 ? 16.0 : 5.0);
-    } else { // whole tiles: as long as the CU with the most of them
-        const int cus = device_cus();
-        const double ktile = (double)((tiles + cus - 1) / cus) * t.bm * t.bn * 32 / t.rate / (kF32MacsPerUs / 256);
-        *us = (d.K + 31) / 32 * (ktile > kF32KTileUs ? ktile : kF32KTileUs) + 5.0;
+    const int cus = device_cus(), nk = (d.K + 31) / 32;
+    const double ktile = t.bm * t.bn * 32 / t.rate / (kF32MacsPerUs / 256); // of a CU's time
+    auto step = [&](double tiles_per_cu) { return ktile * tiles_per_cu > kF32KTileUs ? ktile * tiles_per_cu : kF32KTileUs; };
+    const double mem = ms_mem_us(d), launch = 2.2 + 1.3 * t.bm * t.bn / (128 * 128); // with the store of a tile
+    if (may_split && sk_splits(nk, tiles, 2 * cus)) {
+        // Whole rounds of two tiles per CU, then the rest in ranges of k-tiles, and the hand-over.
+        const int64_t dp = tiles > 2 * cus ? tiles / (2 * cus) * (2 * cus) : 0, iters = (tiles - dp) * nk;
+        const int64_t wgs = std::max<int64_t>(1, std::min({iters / 8, (int64_t)2 * cus, 32 * (tiles - dp)}));
+        const double k = (double)dp / cus * nk * ktile + (double)iters / wgs * step(std::max(1.0, (double)wgs / cus));
+        const double pieces = (double)wgs / (tiles - dp);
+        *us = std::max(k, mem) + launch + (pieces > 1.0 ? 9.0 + 0.2 * pieces : 0.0);
+    } else {
+        *us = std::max(nk * step((double)((tiles + cus - 1) / cus)), mem) + launch + 1.65 * (double)((tiles - 1) / (2 * cus));
     }
     return best;
 }
@@ -82,14 +90,21 @@ int pick_f32_tile(const GemmDesc& d, bool may_split, double* us) {
 // large tiles split over K leave their time in the hand-over.  fp32, us, tiles above -> multi-stage:
 // [1024]^3 37.9 -> 23.5, [1001,776]@[776,1004] 28 -> 20.5, [2574,1316]@Wt[1316,320] 40.7 -> 27.9,
 // [128,640]@Wt[640,1024] 13.2 -> 8.5, [512]^3 -> 9.3; [2592,2048]@[2048,4096] 343 against 347 there.
-// Prices as in gemm_ms_impl.h (32 k per k-tile; the matrix cores' time bounds these).
-constexpr MsTile kF32MsTiles[2] = {{32, 64, 3, 2.5, 2.0, 0.46, 0.94, 3.0, 0.25}, {64, 64, 3, 2.5, 2.6, 0.65, 1.65, 3.0, 0.25}};
+// Both prices (as in gemm_ms_impl.h, 32 k per k-tile; the matrix cores' time bounds these) are fitted to
+// 1,145 random fp32 calls (1 to 60,000 rows, 4 to 125,000 k) timed on the tiles above and on each of these whole
+// and split: 2 % from the fastest on average.  Where a call is bound by its output, or is one or two k-tiles on
+// large tiles, the tiles above win (us, there / here): [11,32]@Wt[32,26480] 3.8 / 4.9, [96,64]@[64,26512] 7.8 /
+// 11.1, [25008,8]@[8,4] 4.1 / 5.9, [43376,32]@Wt[32,16] 5.4 / 7.0, [34704,304]@Wt[304,31] 17.2 / 21.2; but
+// [504,4]@Wt[4,164] 5.2 / 4.0.
+constexpr MsTile kF32MsTiles[2] = {{32, 64, 3, 2.1, 2.5, 1.0, 0.47, 0.91, 3.0, 0.25}, {64, 64, 3, 2.9, 3.4, 1.0, 0.63, 1.56, 3.0, 0.25}};
 
 int run_f32_ms(const GemmDesc& d, hipStream_t stream, bool may_alloc, double other_us) { // 1: not cheaper
     const int am = pick_mode(d.A, d.M, d.K, d.sa_m, d.sa_k, d.sa_b, d.batch, 4, 128, d.pad_a), bm = f32_b_mode(d);
     if (am == LOAD_GENERIC || bm == LOAD_GENERIC) return 1;
     const bool ok[2] = {am == LOAD_KCONTIG, true};
-    const MsPlan plan = ms_plan(d, (d.K + 31) / 32, kF32MsTiles, ok, 2, may_alloc);
+    // N-contiguous B is read in pieces of 256 bytes, half of what the 128-column tiles read: streamed from memory
+    // that costs about a tenth ([25,7616]@[7616,12640] 82 to 94 us here, 78 on tiles of 32x128).
+    const MsPlan plan = ms_plan(d, (d.K + 31) / 32, kF32MsTiles, ok, 2, may_alloc, bm == LOAD_MNCONTIG ? 1.1 : 1.0);
     if (plan.us >= other_us) return 1;
 #define TV_MS(TILE_, BM_, WM_, WN_, NST_, A_, B_) \
     if (plan.tile == TILE_ && am == A_ && bm == B_) return run_ms_cfg<GemmCfg<float, BM_, 64, WM_, WN_, A_, B_>, NST_>(d, stream, plan);

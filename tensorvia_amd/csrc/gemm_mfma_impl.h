@@ -863,6 +863,13 @@ static int sk_grid() {
     });
 }
 
+// Whether the stream-K launch below takes `tiles` tiles of nk k-tiles on G resident workgroups.
+static bool sk_splits(int nk, int64_t tiles, int G) {
+    if (nk < 8) return false;
+    if (nk < 32 && tiles >= G / 2) return false; // G / 2: about one tile per CU
+    return tiles % G != 0;                       // whole rounds: nothing to split
+}
+
 // The stream-K launch: K of at least 32 k-tiles (8 when the tiles do not fill the CUs), at least 8
 // k-tiles per workgroup, and a last round that the resident workgroups do not fill.  Measured
 // against one workgroup per tile with random fp32 inputs (same box, settled clocks): c1
@@ -876,11 +883,8 @@ static int sk_grid() {
 template <class C, bool FUSED>
 static int run_cfg_sk(const GemmDesc& d, hipStream_t stream, int group_m, int tiles_m, int tiles_n, int64_t ntiles, int c_vec) {
     const int nk = (d.K + C::BK - 1) / C::BK;
-    if (nk < 8) return 1;
     int G = sk_grid<C>();
-    if (G <= 0) return 1;
-    if (nk < 32 && ntiles >= G / 2) return 1; // G / 2: about one tile per CU
-    if (ntiles % G == 0) return 1;            // whole rounds: nothing to split
+    if (G <= 0 || !sk_splits(nk, ntiles, G)) return 1;
     // Whole rounds of G tiles run whole; only the last, partial round is split.
     const int64_t dp = ntiles > G ? ntiles / G * G : 0;
     const int64_t iters = (ntiles - dp) * nk;

@@ -263,12 +263,12 @@ void gemm_ms_kernel(GemmDesc d, int tiles_m, int tiles_n, int group_m, int c_vec
 // Host side: the tile and the split of one call.
 
 // A tile as the plan prices it, in us: `fixed` for a launch (first loads, the store), `round` more for
-// each further round of workgroups, t1 per k-tile for a workgroup that has its CU to itself and tr
+// each further round of workgroups, `share` for a CU's second and third workgroup, t1 per k-tile for a workgroup that has its CU to itself and tr
 // when `occ` of them share it (all CUs busy); a split (where it can: s0 >= 0) costs s0 plus s1 per
 // segment of a tile (slots written, the hand-over, the last segment's sums).
 struct MsTile {
     int bm, bn, occ;
-    double fixed, round, t1, tr, s0, s1;
+    double fixed, round, share, t1, tr, s0, s1;
 };
 struct MsPlan {
     int tile = -1; // index into the tile list
@@ -278,13 +278,17 @@ struct MsPlan {
 };
 constexpr double kMsBytesPerUs = 5.0e6; // what the largest streams of these calls reach
 
-// The cheapest of `tiles` (those with ok set) for nk k-tiles of d.
-static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool* ok, int n, bool may_split) {
-    const int cus = device_cus();
+// The least time of d's operands and result in memory, each read or written once.
+static double ms_mem_us(const GemmDesc& d) {
     const double b = d.batch;
-    const double bytes = ((d.sa_b ? b : 1) * d.M + (d.sb_b ? b : 1) * d.N) * d.K * (double)dtype_size(d.dtype_a) +
-                         b * d.M * d.N * (double)dtype_size(d.dtype_c);
-    const double mem = bytes / kMsBytesPerUs;
+    return (((d.sa_b ? b : 1) * d.M + (d.sb_b ? b : 1) * d.N) * d.K * (double)dtype_size(d.dtype_a) +
+            b * d.M * d.N * (double)dtype_size(d.dtype_c)) / kMsBytesPerUs;
+}
+
+// The cheapest of `tiles` (those with ok set) for nk k-tiles of d.
+static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool* ok, int n, bool may_split, double mem_scale = 1.0) {
+    const int cus = device_cus();
+    const double mem = ms_mem_us(d) * mem_scale;
     MsPlan best;
     for (int i = 0; i < n; ++i) {
         if (!ok[i]) continue;
@@ -303,13 +307,15 @@ static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool
         const int64_t full = nt / slots, rest = nt % slots;
         // A CU's second and third workgroup start beside the first, not for nothing (fp16
         // [13][128,512]@[512,928] on 390 tiles of 64x64 11.2 us, 9.4 on 128x128).
-        const double start = t.s0 < 0 || t.occ == 1 || nt <= cus ? 0.0 : 1.5 * (double)((nt < slots ? (nt + cus - 1) / cus : t.occ) - 1);
+        const double start = t.occ == 1 || nt <= cus ? 0.0 : t.share * (double)((nt < slots ? (nt + cus - 1) / cus : t.occ) - 1);
         offer(nt, false, nk * (full * step(slots) + (rest ? step(rest) : 0)), start + t.round * (double)(full + (rest != 0) - 1));
         if (!may_split || t.s0 < 0 || nt > 0x3FFFFFFF / (nk > 0 ? nk : 1)) continue;
         for (int s = 2; s <= 64 && nt * s <= slots && nk >= 2 * s; s += s < 8 ? 1 : s / 4)
             offer(nt * s, true, (double)nk / s * step(nt * s), t.s0 + t.s1 * s);
-        // A range of equal length for every workgroup that the CUs hold: most tiles in two pieces.
-        if (nt * nk >= 4 * slots && rest != 0)
+        // A range of equal length for every workgroup that the CUs hold: most tiles in two pieces.  Not on
+        // 32x64 tiles, three per CU, which read the operands from L2 too often (fp32 [224,59008]@Wt[59008,462] 181 us,
+        // 136 on 64x64).
+        if (t.bm > 32 && nt * nk >= 4 * slots && rest != 0)
             offer(slots, true, (double)nt * nk / slots * step(slots), t.s0 + t.s1 * (2 + (double)slots / nt) + t.round * (double)(full + 1));
     }
     return best;
@@ -367,10 +373,10 @@ static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan)
 // two workgroups per CU, which start faster (bf16 [8][512,96]@Kt[96,512] 5.0 us against 6.2 here), and
 // 256x256 tiles (bf16 [4096]^3 98 us).
 enum { MS_32x64, MS_64x64, MS_64x128, MS_128x128, MS_256x128, MS_DMA_128, MS_DMA_256, MS_TILES };
-constexpr MsTile kMsTiles[MS_TILES] = {{32, 64, 3, 3.5, 2.0, 0.25, 0.43, 3.0, 0.25},  {64, 64, 2, 4.8, 2.6, 0.25, 0.43, 3.0, 0.25},
-                                       {64, 128, 1, 5.0, 3.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.58, 0.58, 5.0, 0.6},
-                                       {256, 128, 1, 6.5, 5.5, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.67, 0.95, -1, 0},
-                                       {256, 256, 1, 9.0, 7.0, 1.3, 1.3, -1, 0}};
+constexpr MsTile kMsTiles[MS_TILES] = {{32, 64, 3, 3.5, 2.0, 1.5, 0.25, 0.43, 3.0, 0.25},  {64, 64, 2, 4.8, 2.6, 1.5, 0.25, 0.43, 3.0, 0.25},
+                                       {64, 128, 1, 5.0, 3.0, 0.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.0, 0.58, 0.58, 5.0, 0.6},
+                                       {256, 128, 1, 6.5, 5.5, 0.0, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.0, 0.67, 0.95, -1, 0},
+                                       {256, 256, 1, 9.0, 7.0, 0.0, 1.3, 1.3, -1, 0}};
 
 // Runs d on the cheapest tile; 1 if that is the 256x256 one, TV_E_NOMEM as run_ms_cfg.  am / bm: the operands' (vector) load modes.
 template <typename T>

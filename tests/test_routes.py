@@ -35,3 +35,15 @@ def test_fp32_few_long_tiles_without_a_workspace(shape):
     M, K, N = shape
     for r in run(call(M, K, N, FLOAT32, entry="noalloc"), "capture 1", call(M, K, N, FLOAT32)):
         assert r.rc == 0 and r.kernel.startswith("gemm_ms_kernel<GemmCfg<float")
+
+
+# fp32 calls that the multi-stage kernel made slower (one or two k-tiles; bound by the output), and ones it serves.
+@pytest.mark.parametrize("shape,bt,kernel", [((11, 32, 26480), True, "gemm_mfma_kernel"), ((96, 64, 26512), False, "gemm_mfma_kernel"),
+                                             ((25008, 8, 4), False, "gemm_mfma_kernel"), ((43376, 32, 16), True, "gemm_mfma_kernel"),
+                                             ((9472, 160, 96), False, "gemm_mfma_kernel"), ((1024, 1024, 1024), False, "gemm_ms_kernel"),
+                                             ((128, 4096, 128), False, "gemm_ms_kernel"), ((2592, 2048, 4096), False, "gemm_mfma_sk_kernel"),
+                                             ((224, 59008, 460), True, "gemm_ms_kernel<GemmCfg<float,64,64")], ids=str)
+def test_fp32_kernel_by_price(shape, bt, kernel):
+    M, K, N = shape
+    r, = run(call(M, K, N, FLOAT32, bt=bt))
+    assert r.rc == 0 and r.kernel.startswith(kernel)
