@@ -295,10 +295,13 @@ static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool
         const MsTile& t = tiles[i];
         const int64_t nt = (int64_t)((d.M + t.bm - 1) / t.bm) * ((d.N + t.bn - 1) / t.bn) * d.batch;
         const int64_t slots = (int64_t)cus * t.occ;
-        // us per k-tile with w workgroups in flight
+        // us per k-tile with w workgroups in flight.  The two-stage tiles' time grows by half of what a full second
+        // workgroup per CU costs as soon as any CU has two, and with their number (K = 4096, bf16: 258 tiles 56 us,
+        // 512 77).
         auto step = [&](int64_t w) {
-            const int64_t load = (w + cus - 1) / cus;
-            return t.occ == 1 || load <= 1 ? t.t1 : t.t1 + (t.tr - t.t1) * (double)(load - 1) / (t.occ - 1);
+            const double load = (double)((w + cus - 1) / cus - 1);
+            if (t.occ == 1 || load <= 0) return t.t1;
+            return t.t1 + (t.tr - t.t1) * (t.s0 < 0 ? 0.5 * load + 0.5 * ((double)w / cus - 1) : load) / (t.occ - 1);
         };
         auto offer = [&](int64_t wgs, bool split, double k_us, double more) {
             const double us = t.fixed + (k_us > mem ? k_us : mem) + more;
@@ -374,8 +377,8 @@ static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan)
 // 256x256 tiles (bf16 [4096]^3 98 us).
 enum { MS_32x64, MS_64x64, MS_64x128, MS_128x128, MS_256x128, MS_DMA_128, MS_DMA_256, MS_TILES };
 constexpr MsTile kMsTiles[MS_TILES] = {{32, 64, 3, 3.5, 2.0, 1.5, 0.25, 0.43, 3.0, 0.25},  {64, 64, 2, 4.8, 2.6, 1.5, 0.25, 0.43, 3.0, 0.25},
-                                       {64, 128, 1, 5.0, 3.0, 0.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.0, 0.58, 0.58, 5.0, 0.6},
-                                       {256, 128, 1, 6.5, 5.5, 0.0, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.0, 0.67, 0.95, -1, 0},
+                                       {64, 128, 1, 5.6, 3.0, 0.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.0, 0.58, 0.58, 5.0, 0.6},
+                                       {256, 128, 1, 6.5, 5.5, 0.0, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.0, 0.67, 1.0, -1, 0},
                                        {256, 256, 1, 9.0, 7.0, 0.0, 1.3, 1.3, -1, 0}};
 
 // Runs d on the cheapest tile; 1 if that is the 256x256 one, TV_E_NOMEM as run_ms_cfg.  am / bm: the operands' (vector) load modes.
@@ -385,12 +388,27 @@ static int run_modes_ms(const GemmDesc& d, hipStream_t stream, int group_m, int 
     const int nk = (d.K + 128 / (int)sizeof(T) - 1) / (128 / (int)sizeof(T));
     // Layouts: 32 rows K-contiguous only; 64 rows M/N-contiguous at 16 bits only (DmaOperand).
     const bool r64a = am == LOAD_KCONTIG || !kI8, r64b = bm == LOAD_KCONTIG || !kI8;
-    // Tall calls whose tiles stream A in rows of k with a pitch of whole 2 KB, more than 64 columns wide
-    // and enough of them for 256x128 tiles: that tile, rotated, whatever the prices (bf16 [65536,2048]@[2048,128] 57 us, 62 on
-    // 128x128 tiles; 74 unrotated, on the two-stage 128x128 tiles as well).
+    // Two shapes outside the prices, measured on 450 calls of 16,384 to 131,072 rows or columns, K of 64 to 8192:
+    //  * Tall: A streamed in rows of whole 4 KB by tiles of one column (N above 64, in batches from 96), at least
+    //    one 256x128 tile per CU, up to 512 MB of A: 256x128, rotated.  us, 256x128 rotated / 128x128: bf16
+    //    [65536,2048]@[2048,128] 42.2 / 49.6, [131072,2048]@[2048,72] 114 / 132, [65536,4096]@[4096,128] 107 / 128,
+    //    32 batches of [2048,2048] with a [2048,128] each 53.6 / 58.5.  Outside: 3072 k (6 KB) 86.5 / 83.9 at N = 96, 16 batches of
+    //    [4096,2048] with 80 columns each 51.0 / 45.2, 50,000 rows (0.77 tiles per CU) 43.3 / 35.0, [131072,4096]
+    //    (1 GB) 213 / 200.
+    //  * Strip: one row or column of 256x256 tiles, where 128x128 tiles would be more than the CUs hold and read the
+    //    large operand twice: 256x256.  us, 256x256 / 128x128: bf16 [224,384]@[384,49184] 15.3 / 23.0, [256,1024]@
+    //    [1024,40960] 25.9 / 29.5, [131072,1152]@[1152,256] 81.8 / 108, int8 [49152,6144]@[6144,256] 82.8 / 112, 256
+    //    batches of [160,1024]@[1024,160] 33.0 / 35.0; not where the second round is less than half full
+    //    ([76512,880]@[880,176], 299 tiles: 59.2 / 46.9), nor for little more than 128 columns ([131072,256]@[256,136]
+    //    40.2 / 30.4) or few k-tiles of a tall one (56 batches of [2960,136]@[136,200] 66.1 / 40.8).
+    const int64_t cus = device_cus();
     const int64_t tall_m = ((int64_t)d.M + 255) / 256 * d.batch, tall_n = (d.N + 127) / 128;
-    const bool tall = d.N > 64 && nk >= 8 && d.sa_m * (int64_t)sizeof(T) % 2048 == 0 && tall_m * tall_n * 4 >= 3 * (int64_t)device_cus() &&
-                      ms_rotation(d, (int)sizeof(T), am, tall_m, tall_n);
+    const bool tall = d.N > (d.batch > 1 ? 95 : 64) && d.N <= 128 && nk >= 8 && d.sa_m * (int64_t)sizeof(T) % 4096 == 0 && tall_m >= cus &&
+                      (int64_t)d.M * d.batch * d.sa_m * (int64_t)sizeof(T) <= (int64_t)512 << 20 && ms_rotation(d, (int)sizeof(T), am, tall_m, tall_n);
+    const int64_t nt128 = ((int64_t)d.M + 127) / 128 * tall_n * d.batch, nt256 = tall_m * ((d.N + 255) / 256);
+    const bool strip = d.M >= 144 && d.N >= 160 && (d.M <= 256 || (d.N <= 256 && nk >= 8)) && nt128 > 2 * cus &&
+                       (nt256 <= cus || nt256 * 4 >= (nt256 + cus - 1) / cus * cus * 3);
+    if (strip) return 1;
     // 32x64 tiles up to one per CU: more of them read B from L2 too often (fp16 [3][128,448]@[448,2744],
     // 516 tiles, 12.7 us; 9.2 on 64x64 or 128x128).
     const bool few32 = ((int64_t)d.M + 31) / 32 * (((int64_t)d.N + 63) / 64) * d.batch <= device_cus();

@@ -47,3 +47,20 @@ def test_fp32_kernel_by_price(shape, bt, kernel):
     M, K, N = shape
     r, = run(call(M, K, N, FLOAT32, bt=bt))
     assert r.rc == 0 and r.kernel.startswith(kernel)
+
+
+# 16-bit and int8 calls outside the tiles' prices: one row or column of 256x256 tiles, tall streams of A, and
+# calls beside each rule's limits.
+@pytest.mark.parametrize("M,K,N,kw,kernel", [
+    (224, 384, 49184, {}, "256,256"), (256, 1024, 40960, dict(bt=True), "256,256"), (131072, 1152, 256, {}, "256,256"),
+    (160, 1024, 160, dict(batch=256), "256,256"), (76512, 880, 176, {}, "128,128"), (131072, 256, 136, {}, "128,128"),
+    (2960, 136, 200, dict(batch=56), "128,128"),
+    (65536, 2048, 128, {}, "256,128"), (131072, 2048, 72, {}, "256,128"), (65536, 4096, 128, {}, "256,128"),
+    (2048, 2048, 128, dict(batch=32), "256,128"), (4096, 2048, 80, dict(batch=16), "128,128"), (50000, 2048, 128, {}, "128,128"),
+    (65536, 3072, 96, {}, "128,128"), (131072, 4096, 128, {}, "128,128"), (65536, 2048, 256, {}, "256,256")],
+    ids=lambda v: "x".join(f"{a}{b}" for a, b in v.items()) if isinstance(v, dict) else str(v))
+def test_tall_and_strip_calls(M, K, N, kw, kernel):
+    r, = run(call(M, K, N, BFLOAT16, **kw))
+    assert r.rc == 0 and f"GemmCfg<__bf16,{kernel}," in r.kernel
+    if (N % 128 == 0 or N == 72) and kernel == "256,128":
+        assert r.kernel.startswith("gemm_ms_kernel")
