@@ -7,22 +7,29 @@
 // the vector units and stored.  16-bit sums run in fused fp32 chains of 32 k, added in order, fp32 ones in
 // fp64 (as cheap here, and at few k the matrix cores' four products per rounding are not to be lost);
 // int8 is exact.
-// Measured on random calls of 1 to 96 rows, columns and k, us a call back to back: bf16 [48,10]@[10,7]
-// 8.6 -> 3.5, fp32 [34,6]@[6,91] 9.1 -> 3.0, [70,6]@[6,38] in a batch of 3 9.6 -> 3.1, int8 [72,14]@[14,1]
-// 13.7 -> 2.9; an empty launch takes about 2.3.
+// K of at most 32 or 64 has its own instantiation: with 128 k laid out whatever K, threads along k loaded 16
+// elements of which K = 16 used two, and the workgroup held 37 KB of LDS (fp32): fp32 [198][10,32]@Wt[32,48] 5.6 us, bf16 [102]
+// [16,16]@Wt[16,80] 4.9, where the kernels of 128 rows took 3.5.
+// Measured on 500 random calls of 1 to 128 rows, columns and k (in a captured graph; an empty launch takes about 2.3 us),
+// the geometric mean of this kernel's time over that of the kernels that serve the call without it:
+//   K            1-32   33-64   65-128
+//   unaligned    0.33   0.41    0.40    (fp32 0.36, 0.50, 0.36; 16-bit 0.37, 0.42, 0.46; int8 0.25, 0.28, 0.33)
+//   aligned      0.71   0.87    1.20    (fp32 0.72, 0.86, 1.11; 16-bit 0.75, 1.00, 1.39; int8 0.63, 0.81, 1.12)
 #include "tv_kernels.h"
 
 namespace tvk {
 namespace tiny {
 
-constexpr int kTile = 16, kMaxK = 128, kPitchA = kMaxK + 4, kPitchB = kTile + 4;
+constexpr int kTile = 16, kMaxK = 128, kPitchB = kTile + 4;
 constexpr int kMaxDim = 128;
 
-template <typename T, typename Acc>
+// KM: the most k (32, 64 or 128): what K does not need is neither loaded nor laid out.
+template <typename T, typename Acc, int KM>
 __global__ __launch_bounds__(256) void gemm_tiny_kernel(GemmDesc d, int tiles_m, int tiles_n) {
     typedef Acc Acc4 __attribute__((ext_vector_type(4)));
-    __shared__ __attribute__((aligned(32))) Acc sa[kTile][kPitchA]; // zero past K and past the rows
-    __shared__ __attribute__((aligned(32))) Acc sb[kMaxK][kPitchB];
+    constexpr int NE = KM / 16; // elements per thread and operand
+    __shared__ __attribute__((aligned(32))) Acc sa[kTile][KM + 4]; // zero past K and past the rows
+    __shared__ __attribute__((aligned(32))) Acc sb[KM][kPitchB];
     const int tid = threadIdx.x;
     const int b = blockIdx.x / (tiles_m * tiles_n), t = blockIdx.x - b * tiles_m * tiles_n;
     const int m0 = t / tiles_n * kTile, n0 = t % tiles_n * kTile;
@@ -30,21 +37,21 @@ __global__ __launch_bounds__(256) void gemm_tiny_kernel(GemmDesc d, int tiles_m,
     const T* B = static_cast<const T*>(d.B) + (int64_t)b * d.sb_b + (int64_t)n0 * d.sb_n;
     // Element e of a thread: consecutive threads along k where k is contiguous, along the rows otherwise.
     const bool ka = d.sa_k == 1, kb = d.sb_k == 1;
-    auto k_of = [&](bool kfast, int e) { return kfast ? tid & (kMaxK - 1) : (tid >> 4) + 16 * e; };
-    auto r_of = [&](bool kfast, int e) { return kfast ? (tid >> 7) + 2 * e : tid & (kTile - 1); };
-    T ra[8], rb[8];
+    auto k_of = [&](bool kfast, int e) { return kfast ? tid & (KM - 1) : (tid >> 4) + 16 * e; };
+    auto r_of = [&](bool kfast, int e) { return kfast ? tid / KM + 256 / KM * e : tid & (kTile - 1); };
+    T ra[NE], rb[NE];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < NE; ++e) {
         const int k = k_of(ka, e), r = r_of(ka, e);
         ra[e] = m0 + r < d.M && k < d.K ? A[r * d.sa_m + k * d.sa_k] : T(0);
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < NE; ++e) {
         const int k = k_of(kb, e), r = r_of(kb, e);
         rb[e] = n0 + r < d.N && k < d.K ? B[r * d.sb_n + k * d.sb_k] : T(0);
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < NE; ++e) {
         sa[r_of(ka, e)][k_of(ka, e)] = static_cast<Acc>(ra[e]);
         sb[k_of(kb, e)][r_of(kb, e)] = static_cast<Acc>(rb[e]);
     }
@@ -88,17 +95,21 @@ __global__ __launch_bounds__(256) void gemm_tiny_kernel(GemmDesc d, int tiles_m,
 int launch_gemm_tiny(const GemmDesc& d, hipStream_t stream) {
     if ((d.bias != nullptr || d.act != TV_ACT_NONE) && d.sc_n != 1) return TV_E_UNSUPPORTED; // as the other kernels
     if (d.M > tiny::kMaxDim || d.N > tiny::kMaxDim || d.K > tiny::kMaxK || d.K < 1) return TV_E_UNSUPPORTED;
-    // Operands in whole 16-byte rows have the direct-load kernels, which are faster from 32 k on (bf16
-    // [8][64,80]@[80,64] 4.9 us, 5.5 here).
+    // Operands in whole 16-byte rows have the direct-load kernels, which are faster above 64 k (16-bit: as fast
+    // from 33 k; the table above).
     const int es = (int)dtype_size(d.dtype_a);
-    if (d.K > 32 && pick_mode(d.A, d.M, d.K, d.sa_m, d.sa_k, d.sa_b, d.batch, es, 256, false) != LOAD_GENERIC &&
+    if (d.K > (es == 2 ? 32 : 64) && pick_mode(d.A, d.M, d.K, d.sa_m, d.sa_k, d.sa_b, d.batch, es, 256, false) != LOAD_GENERIC &&
         pick_mode(d.B, d.N, d.K, d.sb_n, d.sb_k, d.sb_b, d.batch, es, 256, false) != LOAD_GENERIC)
         return TV_E_UNSUPPORTED;
     const int tm = (d.M + 15) / 16, tn = (d.N + 15) / 16;
     const int64_t blocks = (int64_t)tm * tn * d.batch;
     if (blocks > 4 * (int64_t)device_cus()) return TV_E_UNSUPPORTED;
-#define TV_TINY(T_, ACC_) \
-    hipLaunchKernelGGL((tiny::gemm_tiny_kernel<T_, ACC_>), dim3((unsigned)blocks), dim3(256), 0, stream, d, tm, tn); \
+#define TV_TINY_K(T_, ACC_, KM_) \
+    hipLaunchKernelGGL((tiny::gemm_tiny_kernel<T_, ACC_, KM_>), dim3((unsigned)blocks), dim3(256), 0, stream, d, tm, tn)
+#define TV_TINY(T_, ACC_)                          \
+    if (d.K <= 32) TV_TINY_K(T_, ACC_, 32);        \
+    else if (d.K <= 64) TV_TINY_K(T_, ACC_, 64);   \
+    else TV_TINY_K(T_, ACC_, 128);                 \
     return hipGetLastError();
     switch (d.dtype_a) {
         case TV_FLOAT32: TV_TINY(float, double)
@@ -108,6 +119,7 @@ int launch_gemm_tiny(const GemmDesc& d, hipStream_t stream) {
         default: return TV_E_UNSUPPORTED;
     }
 #undef TV_TINY
+#undef TV_TINY_K
 }
 
 } // namespace tvk

@@ -49,7 +49,7 @@ std::string demangled(const char* name) {
     char* s = abi::__cxa_demangle(m.c_str(), nullptr, nullptr, &status);
     std::string r = status == 0 && s ? s : name;
     free(s);
-    for (const char* drop : {"tvk::", "void ", " "}) // "gemm_ms_kernel<GemmCfg<...>,4,false>(GemmDesc,...)"
+    for (const char* drop : {"tvk::", "tiny::", "simt::", "f64::", "void ", " "}) // "gemm_ms_kernel<GemmCfg<...>,4,false>(GemmDesc,...)"
         for (size_t at; (at = r.find(drop)) != std::string::npos;) r.erase(at, std::strlen(drop));
     return r.substr(0, r.find('('));
 }

@@ -143,6 +143,18 @@ def test_smallest_products_exact(hip, dt, shape):
     np.testing.assert_array_equal(to_storage(c.contiguous()), want)
 
 
+@pytest.mark.parametrize("dt", DTYPES, ids=["fp32", "bf16", "fp16", "int8"])
+@pytest.mark.parametrize("K", [31, 32, 33, 48, 63, 64, 65, 128])
+def test_smallest_products_by_k_exact(hip, dt, K):
+    """Each of the 16 x 16-block kernel's instantiations (up to 32, 64 and 128 k) at its edges, aligned and
+    unaligned rows, more blocks than CUs."""
+    for B, M, N in ((1, 17, 48), (1, 33, 47), (40, 20, 96)):
+        x, y = _ints(M + K, (B, M, K)), _ints(N + K, (B, K, N))
+        want = _enc(np.matmul(x.astype(np.float64), y.astype(np.float64)), dt)
+        for at, bt in ((False, False), (False, True), (True, False)):
+            np.testing.assert_array_equal(to_storage(hip.gemm(_dev(x, dt, at), _dev(y, dt, bt))), want)
+
+
 @pytest.mark.parametrize("dt", [FLOAT32, BFLOAT16, INT8], ids=["fp32", "bf16", "int8"])
 @pytest.mark.parametrize("shape", [(64, 64, 8192), (48, 1216, 3712), (65, 77, 2049)], ids=lambda s: "x".join(map(str, s)))
 def test_cold_capture_exact(hip, dt, shape):

@@ -64,3 +64,14 @@ def test_tall_and_strip_calls(M, K, N, kw, kernel):
     assert r.rc == 0 and f"GemmCfg<__bf16,{kernel}," in r.kernel
     if (N % 128 == 0 or N == 72) and kernel == "256,128":
         assert r.kernel.startswith("gemm_ms_kernel")
+
+
+@pytest.mark.parametrize("M,K,N,dt,kernel", [
+    (16, 32, 32, FLOAT32, "gemm_tiny_kernel<float,double,32>"), (32, 64, 48, FLOAT32, "gemm_tiny_kernel<float,double,64>"),
+    (32, 68, 48, FLOAT32, "gemm_m"), (32, 66, 48, FLOAT32, "gemm_tiny_kernel<float,double,128>"),
+    (16, 32, 32, BFLOAT16, "gemm_tiny_kernel<__bf16,float,32>"), (16, 40, 32, BFLOAT16, "gemm_m"),
+    (16, 39, 32, BFLOAT16, "gemm_tiny_kernel<__bf16,float,64>"), (40, 64, 32, INT8, "gemm_tiny_kernel<signedchar,int,64>"),
+    (40, 80, 32, INT8, "gemm_"), (129, 16, 16, INT8, "gemm_"), (9, 127, 128, FLOAT16, "gemm_tiny_kernel<_Float16,float,128>")], ids=str)
+def test_smallest_products(M, K, N, dt, kernel):
+    r, = run(call(M, K, N, dt))
+    assert r.rc == 0 and r.kernel.startswith(kernel) and ("tiny" in kernel or "tiny" not in r.kernel)
