@@ -48,9 +48,10 @@
  *   - bf16/fp16 inputs: fp32 accumulation, output bf16/fp16 (GPU-backend convention) or FLOAT32
  *     (the CPU backend's widened result);
  *   - fp32: fp32 accumulation on the fp32 matrix cores;
- *   - fp64: fp64 accumulation on the fp64 matrix cores, in the reference CPU order;
- *   - any other dtype pair: exact restatement of the reference CPU accumulation rules on a
- *     tiled SIMT kernel.
+ *   - fp64: fp64 accumulation in the reference CPU order, on the fp64 matrix cores or, for small
+ *     matrices, a thread per output;
+ *   - any other dtype pair: exact restatement of the reference CPU accumulation rules on SIMT
+ *     kernels.
  *
  * Calls are asynchronous on `hip_stream` (a hipStream_t, NULL = default stream).  The caller
  * keeps A, B and C alive until the stream has executed the work.  The split-K schedules keep their

@@ -165,13 +165,22 @@ __global__ __launch_bounds__(TILE == 64 ? 512 : 256, 2) void gemm_f64_kernel(Gem
 
 } // namespace f64
 
+static __int128 f64_tiles(const GemmDesc& d, int t) {
+    return (__int128)(((int64_t)d.M + t - 1) / t) * (((int64_t)d.N + t - 1) / t) * d.batch;
+}
+
 // 64 x 64 tiles when they give at least three quarters of the CUs one; 32 x 32 below that, where
-// four times the workgroups each do a quarter of the matrix work per load latency.
+// four times the workgroups each do a quarter of the matrix work per load latency, and where the small
+// tiles leave a quarter of the large ones' outputs out (us, 32 x 32 / 64 x 64: [3000][32,64]@[64,32] 33 / 73,
+// [400][96,64]@[64,96] 37 / 45, [3000][64,64]@[64,16] 57 / 75; but [3000][40,64]@[64,40] 107 / 75).
+int f64_tile(const GemmDesc& d) {
+    const __int128 large = f64_tiles(d, 64);
+    return large * 4 >= device_cus() * 3 && f64_tiles(d, 32) > 3 * large ? 64 : 32;
+}
+
 int launch_gemm_f64(const GemmDesc& d, hipStream_t stream) {
-    auto tiles = [&](int t) { return (__int128)(((int64_t)d.M + t - 1) / t) * (((int64_t)d.N + t - 1) / t) * d.batch; };
-    const bool big = tiles(64) * 4 >= device_cus() * 3;
-    const int t = big ? 64 : 32;
-    const __int128 n = tiles(t);
+    const int t = f64_tile(d);
+    const __int128 n = f64_tiles(d, t);
     if (n > 0x7FFFFFFF) { // more tiles than one grid holds: half of the batch at a time
         if (d.batch <= 1) return TV_E_SHAPE;
         GemmDesc lo = d, hi = d;

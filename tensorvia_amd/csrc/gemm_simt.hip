@@ -1,6 +1,6 @@
 // SIMT path for the dtype pairs the matrix cores do not serve (int16/int32/int64 and mixed pairs;
 // fp64 with fp64 runs on gemm_f64.hip).  It restates the reference CPU backend's arithmetic exactly,
-// reading operands through their strides:
+// reading operands through their strides, in 64 x 64 tiles or with a thread per output (each_output):
 //   * fp16/bf16 inputs are widened to fp32 first (src/backend/cpu/mul.cpp:110-111);
 //   * the result type is compute_type of the widened types (mul.cpp:112,
 //     include/core/type_traits.h:270-287);
@@ -276,22 +276,110 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(GemmDesc d, int64_t tile
     }
 }
 
+// One thread per output, for batches of small matrices and thin ones, whose tiles would be mostly empty.  What
+// bounds it is the latency of its loads (16 of them, 8 k, are in flight per thread: 0.05 us per k where all
+// outputs run at once, 0.2 with one pair of loads waited for at a time), then the lines that a wave's loads
+// touch.  Sums run in the order of the tiled kernels: the results are theirs bit for bit.
+template <typename T, typename R, typename S, bool TILED, typename IDX>
+__global__ __launch_bounds__(256) void gemm_each_kernel(GemmDesc d, IDX total) {
+    using P = Common<T, R>;
+    using X = typename Pick<TILED, T, P>::type;
+    const IDX N = (IDX)d.N, M = (IDX)d.M, stride = (IDX)gridDim.x * 256;
+    const int64_t esa = dtype_size(d.dtype_a), esb = dtype_size(d.dtype_b), ska = d.sa_k * esa, skb = d.sb_k * esb;
+    for (IDX o = (IDX)blockIdx.x * 256 + threadIdx.x; o < total; o += stride) {
+        const IDX row = o / N, n = o - row * N, b = row / M, m = row - b * M;
+        const char* pa = static_cast<const char*>(d.A) + ((int64_t)b * d.sa_b + (int64_t)m * d.sa_m) * esa;
+        const char* pb = static_cast<const char*>(d.B) + ((int64_t)b * d.sb_b + (int64_t)n * d.sb_n) * esb;
+        X sum = 0;
+        S res = 0;
+        auto products = [&]<int G>(int k) { // G products from k on, their elements loaded at once
+            Raw<T> ra[G];
+            Raw<R> rb[G];
+            X x[G], y[G];
+            load_raw<T>(d.dtype_a, ra, [&](int e) { return pa + (int64_t)(k + e) * ska; });
+            load_raw<R>(d.dtype_b, rb, [&](int e) { return pb + (int64_t)(k + e) * skb; });
+            widen_raw<T>(d.dtype_a, ra, [&](int e, T v) { x[e] = cvt<X>(v); });
+            widen_raw<R>(d.dtype_b, rb, [&](int e, R v) { y[e] = cvt<X>(v); });
+#pragma unroll
+            for (int e = 0; e < G; ++e) sum = mac<X, X>(sum, x[e], y[e]);
+        };
+        for (int k0 = 0; k0 < d.K; k0 += 64) {
+            const int end = k0 + min(d.K - k0, 64);
+            int k = k0;
+            for (; k + 8 <= end; k += 8) products.template operator()<8>(k);
+            if (k + 4 <= end) products.template operator()<4>(k), k += 4;
+            if (k + 2 <= end) products.template operator()<2>(k), k += 2;
+            if (k < end) products.template operator()<1>(k);
+            if constexpr (TILED) {
+                const S c = cvt<S>(sum);
+                res = k0 == 0 ? c : cvt<S>(add<Common<S, S>>((Common<S, S>)res, (Common<S, S>)c));
+                sum = 0;
+            }
+        }
+        static_cast<S*>(d.C)[(int64_t)b * d.sc_b + (int64_t)m * d.sc_m + (int64_t)n * d.sc_n] = TILED ? res : cvt<S>(sum);
+    }
+}
+
 static int widen(int dt) { return (dt == TV_BFLOAT16 || dt == TV_FLOAT16) ? TV_FLOAT32 : dt; }
+
+// Whether a thread per output is cheaper than a tile per workgroup: every matrix costs at least one whole tile,
+// so batches of small matrices and thin ones pay for 64 x 64 outputs that they do not have (fp64
+// [100000][4,4]@[4,4] 2,156 us on tiles, 11 here; int32 [10000][8,8]@[8,8] 170, 7; fp64 [1000000,3]@[3,3] 356, 22).
+// Both prices, in us, are fitted to 1,800 random calls (1 to 200,000 matrices of 1 to 500,000 rows or columns, K of 1 to
+// 4096) timed both ways: 2.6 % from the cheaper one on average, 9 of them more than 8 % slower than the tiles.
+static bool each_output(const GemmDesc& d) {
+    const double cus = device_cus(), K = d.K, total = (double)d.batch * d.M * d.N;
+    auto tiles = [&](int t) { return (double)(((int64_t)d.M + t - 1) / t) * (double)(((int64_t)d.N + t - 1) / t) * d.batch; };
+    auto over = [](double tiles, double held) { return tiles > held ? tiles / held : 1.0; };
+    // Lanes on consecutive columns of a row-major B share its lines; rows of fewer than a wave's columns take lines
+    // of several rows of A, and a B contiguous along k a line per lane, which the L1 seldom keeps until the next k.
+    const bool b_lines = d.sb_n != 1 && d.N > 1, lines = b_lines || d.N < 64;
+    const double k_us = b_lines ? 0.13 : lines ? 0.089 : 0.058, mac_us = lines ? 1.5e-6 : 0.68e-6;
+    const double each = 1.9 + K * (total * mac_us > k_us ? total * mac_us : k_us);
+    double tile;
+    if (d.dtype_a == TV_FLOAT64 && d.dtype_b == TV_FLOAT64) {
+        const int t = f64_tile(d);
+        const double n = tiles(t) / cus, steps = 2.0 * ((d.K + 63) / 64);
+        tile = t == 64 ? 3.3 + 2.6 * n + steps * (n > 0.8 ? 1.6 * n : 1.3) : 3.3 + 1.6 * n + steps * (n > 0.8 ? 0.57 * n : 0.46);
+    } else {
+        const bool i64 = d.dtype_a == TV_INT64 || d.dtype_b == TV_INT64;
+        const double n = tiles(kTile);
+        tile = 5.0 + 2.75 * (i64 ? 1.8 : 1.0) * K / kBk * over(n, 0.96 * cus) + 3.9 * n / cus;
+    }
+    return each < tile;
+}
+
+template <typename T, typename R, typename S, bool TILED>
+static int launch_each(const GemmDesc& d, hipStream_t stream) {
+    const int64_t total = (int64_t)d.batch * d.M * d.N, blocks = (total + 255) / 256;
+    const unsigned grid = blocks < 65536 ? (unsigned)blocks : 65536u;
+    if (total < ((int64_t)1 << 31))
+        hipLaunchKernelGGL((gemm_each_kernel<T, R, S, TILED, uint32_t>), dim3(grid), dim3(256), 0, stream, d, (uint32_t)total);
+    else
+        hipLaunchKernelGGL((gemm_each_kernel<T, R, S, TILED, int64_t>), dim3(grid), dim3(256), 0, stream, d, total);
+    return hipGetLastError();
+}
 
 template <typename T, typename R>
 static int launch_tr(const GemmDesc& d, hipStream_t stream) {
     using S = decltype(result_value<T, R>());
-    const int64_t tiles_m = ((int64_t)d.M + kTile - 1) / kTile, tiles_n = ((int64_t)d.N + kTile - 1) / kTile;
-    // Up to 2^25 x 2^25 tiles and 2^31 batches: the grid is capped and a workgroup takes every
-    // grid-size-th tile; a count past 2^62 could never run.
-    const __int128 n = (__int128)tiles_m * tiles_n * d.batch;
-    if (n > ((__int128)1 << 62)) return TV_E_SHAPE;
-    const unsigned blocks = n < ((int64_t)1 << 20) ? (unsigned)n : 1u << 20;
-    if ((__int128)d.batch * d.M * d.N >= 1024 * 1024)
-        hipLaunchKernelGGL((gemm_simt_kernel<T, R, S, true>), dim3(blocks), dim3(256), 0, stream, d, tiles_m, tiles_n);
-    else
-        hipLaunchKernelGGL((gemm_simt_kernel<T, R, S, false>), dim3(blocks), dim3(256), 0, stream, d, tiles_m, tiles_n);
-    return hipGetLastError();
+    const bool chunked = (__int128)d.batch * d.M * d.N >= 1024 * 1024; // mul_kernel_tiled
+    if (each_output(d)) return chunked ? launch_each<T, R, S, true>(d, stream) : launch_each<T, R, S, false>(d, stream);
+    if constexpr (__is_same(T, double) && __is_same(R, double)) {
+        return launch_gemm_f64(d, stream);
+    } else {
+        const int64_t tiles_m = ((int64_t)d.M + kTile - 1) / kTile, tiles_n = ((int64_t)d.N + kTile - 1) / kTile;
+        // Up to 2^25 x 2^25 tiles and 2^31 batches: the grid is capped and a workgroup takes every
+        // grid-size-th tile; a count past 2^62 could never run.
+        const __int128 n = (__int128)tiles_m * tiles_n * d.batch;
+        if (n > ((__int128)1 << 62)) return TV_E_SHAPE;
+        const unsigned blocks = n < ((int64_t)1 << 20) ? (unsigned)n : 1u << 20;
+        if (chunked)
+            hipLaunchKernelGGL((gemm_simt_kernel<T, R, S, true>), dim3(blocks), dim3(256), 0, stream, d, tiles_m, tiles_n);
+        else
+            hipLaunchKernelGGL((gemm_simt_kernel<T, R, S, false>), dim3(blocks), dim3(256), 0, stream, d, tiles_m, tiles_n);
+        return hipGetLastError();
+    }
 }
 
 template <typename T>
@@ -304,9 +392,7 @@ static int launch_t(const GemmDesc& d, hipStream_t stream) {
         case TV_INT32: return launch_tr<T, int>(d, stream);
         case TV_INT64: return launch_tr<T, long>(d, stream);
         case TV_FLOAT32: return launch_tr<T, float>(d, stream);
-        case TV_FLOAT64:
-            if constexpr (!__is_same(T, double)) return launch_tr<T, double>(d, stream);
-            else return launch_gemm_f64(d, stream);
+        case TV_FLOAT64: return launch_tr<T, double>(d, stream);
         default: return TV_E_DTYPE;
     }
 }

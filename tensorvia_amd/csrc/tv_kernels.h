@@ -201,6 +201,7 @@ int gemm_sk_workspace(hipStream_t stream, size_t cnt_ints, size_t slot_bytes, in
 int launch_gemm_simt(const GemmDesc& d, hipStream_t stream);
 int launch_gemm_tiny(const GemmDesc& d, hipStream_t stream); // TV_E_UNSUPPORTED above its sizes
 int launch_gemm_f64(const GemmDesc& d, hipStream_t stream); // fp64 x fp64 -> fp64
+int f64_tile(const GemmDesc& d);                            // rows and columns of its tiles for d
 int launch_gemm_k0(const GemmDesc& d, hipStream_t stream); // K = 0: C = epilogue(0)
 int launch_repack(const tv_repack_args* a, hipStream_t stream);
 int launch_typecast(const void* src, int src_dt, void* dst, int dst_dt, int64_t n, hipStream_t stream);

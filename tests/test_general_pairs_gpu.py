@@ -1,5 +1,5 @@
-"""The tiled kernels of the dtype pairs without 8/16/32-bit matrix-core types (gemm_simt.hip,
-gemm_f64.hip) at the edges of their 64- and 32-wide tiles, 32-wide k-steps and 64-wide k-chunks,
+"""The kernels of the dtype pairs without 8/16/32-bit matrix-core types (gemm_simt.hip, gemm_f64.hip): tiles
+at the edges of their 64- and 32-wide tiles, 32-wide k-steps and 64-wide k-chunks, and a thread per output,
 against the oracle's MulImpl<CPU>: row-major, transposed and strided views, batches, broadcast.
 
 Integer pairs equal the oracle bit for bit, wrap-around included.  Float pairs sum the same products
@@ -21,6 +21,9 @@ INT_LIM = {I8: 100, I16: 30000, I32: 2**30, I64: 2**61}
 PAIRS = [(F64, F64), (FLOAT32, BFLOAT16), (FLOAT16, FLOAT32), (BFLOAT16, FLOAT16), (FLOAT32, F64), (I16, I16), (I32, I32),
          (I16, I32), (I8, I64)]
 SHAPES = [(1, 1, 1), (31, 63, 33), (64, 64, 64), (65, 97, 63), (33, 32, 130), (200, 129, 300)]
+# The calls above run a thread per output but for the last; these run on tiles (test_routes.py), 64 x 64 and, in
+# fp64, 32 x 32 up to 191 of the large ones.
+TILED = [(577, 97, 513), (897, 97, 897), (705, 129, 641), (640, 31, 832), (833, 64, 639)]
 LARGE = [(1030, 97, 1021), (1024, 64, 1024)]  # 2^20 outputs and more: 64-wide chunk sums
 
 
@@ -73,6 +76,15 @@ def test_general_pairs_edges(hip, pair, shape):
 
 
 @pytest.mark.parametrize("pair", PAIRS, ids=lambda p: f"{p[0]}x{p[1]}")
+@pytest.mark.parametrize("shape", TILED, ids=lambda s: "x".join(map(str, s)))
+def test_general_pairs_tile_edges(hip, pair, shape):
+    (da, db), (M, K, N) = pair, shape
+    a, b = _values(M + 3 * K, (M, K), da), _values(N + 5 * K, (K, N), db)
+    for la, lb in (("row", "row"), ("trans", "trans"), ("step", "step")):
+        _check(hip, da, db, a, b, _view(a, da, la), _view(b, db, lb))
+
+
+@pytest.mark.parametrize("pair", PAIRS, ids=lambda p: f"{p[0]}x{p[1]}")
 @pytest.mark.parametrize("shape", LARGE, ids=lambda s: "x".join(map(str, s)))
 def test_general_pairs_chunked(hip, pair, shape):
     (da, db), (M, K, N) = pair, shape
@@ -86,3 +98,29 @@ def test_general_pairs_batched(hip, pair):
     a, b, b1 = _values(1, (3, 70, 45), da), _values(2, (3, 45, 66), db), _values(3, (45, 66), db)
     _check(hip, da, db, a, b, _view(a, da, "row"), _view(b, db, "row"))
     _check(hip, da, db, a, b1, _view(a, da, "step"), _view(b1, db, "trans"))
+
+
+@pytest.mark.parametrize("pair", PAIRS, ids=lambda p: f"{p[0]}x{p[1]}")
+def test_general_pairs_small_matrices(hip, pair):
+    """Batches of small matrices and thin ones, a thread per output: every remainder of its groups of 8 k, views,
+    broadcast operands, a column-strided C."""
+    da, db = pair
+    for B, M, K, N in ((300, 4, 5, 3), (64, 1, 130, 1), (40, 5, 71, 7), (200, 3, 8, 9), (90, 2, 1, 2)):
+        a, b = _values(M + 3 * K, (B, M, K), da), _values(N + 5 * K, (B, K, N), db)
+        for la, lb in (("row", "row"), ("trans", "trans"), ("step", "step")):
+            _check(hip, da, db, a, b, _view(a, da, la), _view(b, db, lb))
+        _check(hip, da, db, a, b[0], _view(a, da, "row"), _view(b[0], db, "trans"))
+    a, b = _values(7, (5000, 6), da), _values(8, (6, 3), db)
+    _check(hip, da, db, a, b, _view(a, da, "row"), _view(b, db, "row"))
+    rt = orc.result_type(da, db)
+    c = _view(np.zeros((3, 5000), dtype=orc.NP[rt]), rt, "row").t()
+    hip.gemm(_view(a, da, "row"), _view(b, db, "row"), out=c, out_dtype=rt)
+    np.testing.assert_array_equal(to_storage(c), to_storage(hip.gemm(_view(a, da, "row"), _view(b, db, "row"), out_dtype=rt)))
+
+
+@pytest.mark.parametrize("pair", PAIRS, ids=lambda p: f"{p[0]}x{p[1]}")
+def test_general_pairs_thin_chunked(hip, pair):
+    """2^20 outputs and more with a thread each: 64-wide chunk sums and a last chunk of 3 k."""
+    da, db = pair
+    a, b = _values(11, (350001, 67), da), _values(12, (67, 3), db)
+    _check(hip, da, db, a, b, _view(a, da, "row"), _view(b, db, "row"))

@@ -3,7 +3,7 @@
 import pytest
 
 from tests.routes import call, run
-from tests.util import BFLOAT16, FLOAT16, FLOAT32, INT8
+from tests.util import BFLOAT16, FLOAT16, FLOAT32, FLOAT64, INT8, INT16, INT32
 
 SPLIT = {
     "bf16_prompt": dict(M=333, K=4096, N=11008, dt=BFLOAT16),
@@ -75,3 +75,31 @@ def test_tall_and_strip_calls(M, K, N, kw, kernel):
 def test_smallest_products(M, K, N, dt, kernel):
     r, = run(call(M, K, N, dt))
     assert r.rc == 0 and r.kernel.startswith(kernel) and ("tiny" in kernel or "tiny" not in r.kernel)
+
+
+# fp64, integer and mixed pairs: a thread per output where the tiles would be mostly empty.
+@pytest.mark.parametrize("M,K,N,dt,kw,kernel", [
+    (4, 4, 4, FLOAT64, dict(batch=100000), "gemm_each"), (4, 4, 4, INT32, dict(batch=100000), "gemm_each"),
+    (8, 8, 8, INT16, dict(batch=10000), "gemm_each"), (1000000, 3, 3, FLOAT64, {}, "gemm_each"), (4, 5, 3, FLOAT64, dict(batch=300), "gemm_each"),
+    (350001, 67, 3, FLOAT64, {}, "gemm_each"), (350001, 67, 3, FLOAT32, dict(db=BFLOAT16), "gemm_each"), (5000, 6, 3, INT32, {}, "gemm_each"),
+    (32, 64, 32, FLOAT64, dict(batch=3000), "gemm_f64_kernel<32,"), (40, 64, 40, FLOAT64, dict(batch=3000), "gemm_f64_kernel<64,"),
+    (1000, 1000, 1000, FLOAT64, {}, "gemm_f64_kernel<64,"), (200, 300, 129, FLOAT64, {}, "gemm_f64_kernel<32,"),
+    (1000, 600, 1000, INT32, {}, "gemm_simt_kernel"), (128, 512, 65, FLOAT32, dict(db=BFLOAT16, bt=True), "gemm_simt_kernel"),
+    (512, 600, 512, INT16, {}, "gemm_simt_kernel"), (64, 600, 64, INT16, {}, "gemm_each")], ids=str)
+def test_general_pairs(M, K, N, dt, kw, kernel):
+    for r in run(call(M, K, N, dt, **kw), call(M, K, N, dt, **kw, entry="noalloc")):
+        assert r.rc == 0 and r.kernel.startswith(kernel)
+
+
+def test_general_pairs_tests_run_on_tiles():
+    """The shapes that tests/test_general_pairs_gpu.py runs at the edges of the tiles do run on them."""
+    from tests.test_general_pairs_gpu import LARGE, PAIRS, TILED
+    import oracle as orc
+    for da, db in PAIRS:
+        for M, K, N in TILED + LARGE:
+            for at, bt, step in ((0, 0, 0), (1, 1, 0), (0, 0, 1)):
+                st = dict(sa=(0, 3 * 2 * K, 2), sb=(0, 3 * 2 * N, 2)) if step else dict(at=at, bt=bt)
+                r, = run(call(M, K, N, da, out=orc.result_type(da, db), db=db, **st))
+                assert r.rc == 0 and r.kernel.startswith(("gemm_simt_kernel", "gemm_f64_kernel")), (da, db, M, K, N, r.kernel)
+    kernels = {run(call(M, K, N, FLOAT64))[0].kernel for M, K, N in TILED + LARGE}
+    assert kernels >= {"gemm_f64_kernel<32,false>", "gemm_f64_kernel<64,false>", "gemm_f64_kernel<64,true>"}
