@@ -178,22 +178,33 @@ int f64_tile(const GemmDesc& d) {
     return large * 4 >= device_cus() * 3 && f64_tiles(d, 32) > 3 * large ? 64 : 32;
 }
 
-int launch_gemm_f64(const GemmDesc& d, hipStream_t stream) {
-    const int t = f64_tile(d);
+// chunks: the sum's order, by the whole call's outputs.
+static int launch_tiles(const GemmDesc& d, int t, bool chunks, hipStream_t stream) {
     const __int128 n = f64_tiles(d, t);
-    if (n > 0x7FFFFFFF) { // more tiles than one grid holds: half of the batch at a time
-        if (d.batch <= 1) return TV_E_SHAPE;
+    const int threads = t == 64 ? 512 : 256;
+    if (n * threads > 0xFFFFFFFFll) { // more than one grid holds (2^32 threads): half of the batch or of the rows at a time
         GemmDesc lo = d, hi = d;
-        lo.batch = d.batch / 2;
-        hi.batch = d.batch - lo.batch;
-        hi.A = static_cast<const double*>(d.A) + lo.batch * d.sa_b;
-        hi.B = static_cast<const double*>(d.B) + lo.batch * d.sb_b;
-        hi.C = static_cast<double*>(d.C) + lo.batch * d.sc_b;
-        const int rc = launch_gemm_f64(lo, stream);
-        return rc ? rc : launch_gemm_f64(hi, stream);
+        if (d.batch > 1) {
+            lo.batch = d.batch / 2;
+            hi.batch = d.batch - lo.batch;
+            hi.A = static_cast<const double*>(d.A) + lo.batch * d.sa_b;
+            hi.B = static_cast<const double*>(d.B) + lo.batch * d.sb_b;
+            hi.C = static_cast<double*>(d.C) + lo.batch * d.sc_b;
+        } else if (d.M > t) {
+            lo.M = (d.M / 2 + t - 1) / t * t;
+            hi.M = d.M - lo.M;
+            hi.A = static_cast<const double*>(d.A) + lo.M * d.sa_m;
+            hi.C = static_cast<double*>(d.C) + lo.M * d.sc_m;
+        } else {
+            lo.N = (d.N / 2 + t - 1) / t * t;
+            hi.N = d.N - lo.N;
+            hi.B = static_cast<const double*>(d.B) + lo.N * d.sb_n;
+            hi.C = static_cast<double*>(d.C) + lo.N * d.sc_n;
+        }
+        const int rc = launch_tiles(lo, t, chunks, stream);
+        return rc ? rc : launch_tiles(hi, t, chunks, stream);
     }
     const int tm = (int)(((int64_t)d.M + t - 1) / t), tn = (int)(((int64_t)d.N + t - 1) / t);
-    const bool chunks = (__int128)d.batch * d.M * d.N >= 1024 * 1024;
 #define TV_F64(T_, C_)                                                                                                     \
     if (t == T_ && chunks == C_)                                                                                           \
         hipLaunchKernelGGL((f64::gemm_f64_kernel<T_, C_>), dim3((unsigned)n), dim3(T_ == 64 ? 512 : 256), 0, stream, d, tm, \
@@ -204,6 +215,10 @@ int launch_gemm_f64(const GemmDesc& d, hipStream_t stream) {
     TV_F64(32, false)
 #undef TV_F64
     return hipGetLastError();
+}
+
+int launch_gemm_f64(const GemmDesc& d, hipStream_t stream) {
+    return launch_tiles(d, f64_tile(d), (__int128)d.batch * d.M * d.N >= 1024 * 1024, stream);
 }
 
 } // namespace tvk

@@ -306,3 +306,19 @@ def test_many_small_batches(hip, dt, batch, M, K, N, bcast):
         np.testing.assert_array_equal(got.numpy(), want.astype(np.int64).astype(got.numpy().dtype))
     else:
         np.testing.assert_array_equal(got.to(torch.float64).numpy(), torch.from_numpy(want).to(dt).to(torch.float64).numpy())
+
+
+def test_fp64_more_tiles_than_one_grid(hip):
+    """17,000,001 products of 16 x 16 fp64 (one 32 x 32 tile each, 256 threads: more than the 2^32 threads of one
+    grid), A and B the same for all: every matrix of the result is the one product, exact."""
+    batch, M, K, N = 17_000_001, 16, 200, 16
+    a, b = _ints((M, K), -3, 3, torch.int8, 121).to(torch.float64), _ints((K, N), -3, 3, torch.int8, 122).to(torch.float64)
+    want = torch.from_numpy(np.matmul(a.cpu().numpy(), b.cpu().numpy())).cuda()
+    c = torch.empty((batch, M, N), dtype=torch.float64, device="cuda")
+    c[::1_000_000] = -1.0
+    hip.gemm(a.expand(batch, M, K), b, out=c)
+    torch.cuda.synchronize()
+    for i in range(0, batch, 1_000_000):
+        assert bool((c[i:i + 1_000_000] == want).all())
+    del c
+    torch.cuda.empty_cache()

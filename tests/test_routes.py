@@ -103,3 +103,15 @@ def test_general_pairs_tests_run_on_tiles():
                 assert r.rc == 0 and r.kernel.startswith(("gemm_simt_kernel", "gemm_f64_kernel")), (da, db, M, K, N, r.kernel)
     kernels = {run(call(M, K, N, FLOAT64))[0].kernel for M, K, N in TILED + LARGE}
     assert kernels >= {"gemm_f64_kernel<32,false>", "gemm_f64_kernel<64,false>", "gemm_f64_kernel<64,true>"}
+
+
+@pytest.mark.parametrize("batch,M,K,N", [(9000000, 64, 200, 64), (20000000, 40, 300, 41), (1, 2146435071, 64, 300), (1, 64, 64, 2146435071),
+                                         (8388607, 64, 200, 64)], ids=str)
+def test_fp64_calls_larger_than_one_grid(batch, M, K, N):
+    """More tiles than one grid holds (2^32 threads): several launches that cover the call."""
+    r, = run(call(M, K, N, FLOAT64, batch=batch))
+    assert r.rc == 0 and not any(e[0] == "launch-refused" for e in r.events)
+    t = 64 if "f64_kernel<64" in r.kernel else 32
+    tiles = batch * -(-M // t) * -(-N // t)
+    assert sum(grid for _, grid, _ in r.launches) == tiles and all(k == "gemm_f64_kernel<%d,true>" % t for k, _, _ in r.launches)
+    assert (len(r.launches) == 1) == (tiles * (512 if t == 64 else 256) < 1 << 32)
