@@ -285,7 +285,7 @@ static double ms_mem_us(const GemmDesc& d) {
             b * d.M * d.N * (double)dtype_size(d.dtype_c)) / kMsBytesPerUs;
 }
 
-// The cheapest of `tiles` (those with ok set) for nk k-tiles of d.
+// The cheapest of `tiles` (those with ok set) for nk k-tiles of d; none where no grid of them fits.
 static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool* ok, int n, bool may_split, double mem_scale = 1.0) {
     const int cus = device_cus();
     const double mem = ms_mem_us(d) * mem_scale;
@@ -295,6 +295,7 @@ static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool
         const MsTile& t = tiles[i];
         const int64_t nt = (int64_t)((d.M + t.bm - 1) / t.bm) * ((d.N + t.bn - 1) / t.bn) * d.batch;
         const int64_t slots = (int64_t)cus * t.occ;
+        if (nt * (t.bm * t.bn <= 64 * 64 ? 256 : 512) > 0xFFFFFFFFll) continue; // a grid holds fewer than 2^32 threads
         // us per k-tile with w workgroups in flight.  The two-stage tiles' time grows by half of what a full second
         // workgroup per CU costs as soon as any CU has two, and with their number (K = 4096, bf16: 258 tiles 56 us,
         // 512 77).

@@ -115,3 +115,17 @@ def test_fp64_calls_larger_than_one_grid(batch, M, K, N):
     tiles = batch * -(-M // t) * -(-N // t)
     assert sum(grid for _, grid, _ in r.launches) == tiles and all(k == "gemm_f64_kernel<%d,true>" % t for k, _, _ in r.launches)
     assert (len(r.launches) == 1) == (tiles * (512 if t == 64 else 256) < 1 << 32)
+
+
+@pytest.mark.parametrize("dt", [BFLOAT16, FLOAT16, INT8, FLOAT32], ids=["bf16", "fp16", "int8", "fp32"])
+def test_tallest_calls_fit_one_grid(dt):
+    """2^31 - 2^20 - 1 rows or columns: tiles whose grid would hold 2^32 threads or more are not chosen."""
+    L, lines = 2146435071, []
+    for short, K in ((1, 1), (1, 16), (8, 16), (16, 8), (40, 4), (64, 1)):
+        for M, N in ((L, short), (short, L))[:2 if short > 32 else 1]:  # up to 32 rows: the GEMV
+            for bt in (False, True):
+                lines += [call(M, K, N, dt, bt=bt), call(M, K, N, dt, bt=bt, entry="noalloc")]
+                if dt != INT8:
+                    lines.append(call(M, K, N, dt, bt=bt, act=1))
+    for line, r in zip(lines, run(*lines)):
+        assert r.rc == 0 and r.launches, (line, r)
