@@ -72,7 +72,10 @@ int pick_f32_tile(const GemmDesc& d, bool may_split, double* us) {
     const int cus = device_cus(), nk = (d.K + 31) / 32;
     const double ktile = t.bm * t.bn * 32 / t.rate / (kF32MacsPerUs / 256); // of a CU's time
     auto step = [&](double tiles_per_cu) { return ktile * tiles_per_cu > kF32KTileUs ? ktile * tiles_per_cu : kF32KTileUs; };
-    const double mem = ms_mem_us(d), launch = 2.2 + 1.3 * t.bm * t.bn / (128 * 128); // with the store of a tile
+    // A launch with the store of a tile, which the fused epilogue makes longer here: [232,28]@Wt[28,8184] with bias
+    // and SiLU 16.4 us, 8.6 on the multi-stage tiles.
+    const bool epi = d.bias != nullptr || d.act != TV_ACT_NONE;
+    const double mem = ms_mem_us(d), launch = 2.2 + (epi ? 3.0 : 1.3) * t.bm * t.bn / (128 * 128);
     if (may_split && sk_splits(nk, tiles, 2 * cus)) {
         // Whole rounds of two tiles per CU, then the rest in ranges of k-tiles, and the hand-over.
         const int64_t dp = tiles > 2 * cus ? tiles / (2 * cus) * (2 * cus) : 0, iters = (tiles - dp) * nk;
