@@ -23,11 +23,13 @@ pytestmark = pytest.mark.gpu
 
 # (name, dtype, M, K, N, value range): each uses the per-stream workspace -- a B copied into padded
 # rows (N = 260), an A copied into padded rows (K = 700), a padded W then the split-K GEMV
-# (N = 129), the GEMV's split-K slots, the fp32 stream-K slots (64 tiles) and the int8 stream-K
-# slots (128 tiles of 128x128).
+# (N = 129), the GEMV's split-K slots, the fp32 stream-K slots, the slots of multi-stage tiles split
+# over K in fp32, bf16 and int8 -- but for two that run on whole tiles (fp32 1024^3, int8 512x4096x4096).
 CASES = [("bf16_padded_b", BFLOAT16, 64, 512, 260, 3), ("bf16_padded_a", BFLOAT16, 300, 700, 1024, 3),
          ("bf16_padded_skinny_w", BFLOAT16, 1, 4096, 129, 2), ("bf16_gemv_split_k", BFLOAT16, 8, 4096, 4096, 2),
-         ("fp32_stream_k", FLOAT32, 1024, 1024, 1024, 3), ("int8_stream_k", INT8, 512, 4096, 4096, 127)]
+         ("fp32_stream_k", FLOAT32, 1024, 1024, 1024, 3), ("int8_stream_k", INT8, 512, 4096, 4096, 127),
+         ("fp32_two_stage_split", FLOAT32, 75, 252, 8352, 3), ("fp32_split", FLOAT32, 64, 4096, 64, 3),
+         ("bf16_split", BFLOAT16, 48, 3712, 1216, 2), ("int8_split", INT8, 34, 2192, 1216, 127)]
 THREADS = 4
 ITERS = 6
 

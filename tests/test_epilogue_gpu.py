@@ -10,7 +10,7 @@ widened by the activation's slope (at most 1; the float exp/tanh add a few ulp):
   bf16/fp16 out: |c - ref| <= 1e-2 * |ref| + 1e-5 * sqrt(K) * sum_k |a||b| + 1e-3 (half ulp near 0)
 
 Every kernel family the router can pick is covered: the fp32 MFMA kernel, the 16-bit direct-load
-kernel (bf16, half output and fp32 output; 128x128 and 256x256 tiles), the small-K persistent kernel (fp16, K = 128, >= 1024
+kernels (bf16, half output and fp32 output), the small-K persistent kernel (fp16, K = 128, >= 1024
 tiles) and both GEMV kernels (matrix-core: bf16 at M = 1 and 8; dot-product: fp32, and bf16
 narrower than 64 columns), with per-column, full and batch-broadcast bias.
 """
@@ -160,19 +160,18 @@ def test_streaming_store_repeated(act):
 @pytest.mark.parametrize("act", [tv.ACT_RELU, tv.ACT_SILU])
 @pytest.mark.parametrize("N,bt", [(4104, False), (4100, True)], ids=["N4104", "N4100-Bt"])
 def test_direct_load_256_tiles_fused(act, N, bt):
-    """More 128x128 tiles than fit one round of resident workgroups (561 here): the 16-bit GEMM runs
-    153 tiles of 256x256, with the fused column bias and activation; rows of C in whole 16-byte
-    chunks (N = 4104), or not (N = 4100, B a K-contiguous view so that it still loads directly)."""
+    """More 128x128 tiles than fit one round of resident workgroups (561 here), with the fused column bias
+    and activation; rows of C in whole 16-byte chunks (N = 4104), or not (N = 4100, B a K-contiguous
+    view so that it still loads directly).  The fused 256x256 tiles: tests/test_kernel_cases_gpu.py."""
     run_case(tv.BFLOAT16, tv.BFLOAT16, 0, 2100, 256, N, "col", act, bt=bt, seed=41)
 
 
 @pytest.mark.parametrize("act", [tv.ACT_NONE, tv.ACT_RELU, tv.ACT_SILU, tv.ACT_TANH])
 @pytest.mark.parametrize("bias_kind,dt", [("col", tv.BFLOAT16), ("colb", tv.BFLOAT16), ("none", tv.FLOAT16)])
 def test_two_tiles_per_cu_fused(act, bias_kind, dt):
-    """Two or more 256x256 tiles per CU (8 x 8 x 8 = 512 here, the c3 layout at K = 256), where the
-    plain GEMM chains tiles: the fused call runs one workgroup per tile, with the per-column (per
-    batch) or no bias and the activation applied as the 16-bit output is staged.  Batches 0 and 7
-    are checked against the fp64 composition."""
+    """Eight 128x128 tiles per CU over a batch (8 x 16 x 16 = 2,048), with the per-column (per batch) or
+    no bias and the activation applied as the 16-bit output is staged.  Batches 0 and 7 are checked
+    against the fp64 composition."""
     run_case(dt, dt, 8, 2048, 256, 2048, bias_kind, act, seed=43, check=[0, 7])
 
 

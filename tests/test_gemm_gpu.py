@@ -435,16 +435,11 @@ def test_small_k_row_groups_exact(hip, dt, batch, M, K, N, bt):
                                          (0, 1100, 4104, 2040), (3, 600, 4096, 1280), (0, 1100, 8192, 2040),
                                          (8, 3000, 4096, 64)])
 def test_direct_load_stream_k_bit_exact(hip, dt, batch, M, K, N):
-    """16-bit and int8 GEMMs with few, long tiles (16-bit: 32, 18, 20, 64, 144, 150, 144 and 192
-    tiles of 128x128; int8: 8, 6, 6, 16, 40, 45, 40 and 96 of 256x256; K = 8192, 4096 and the
-    ragged 8208 and 4104) run the direct-load kernel's stream-K schedule: tiles summed in segments
-    by several workgroups.  16-bit 128x128 tiles split at up to half as many tiles as resident
-    workgroups, but above a quarter only into segments of at least 32 k-tiles or on a tile grid of
-    one column: 144 tiles at K = 8192 and 8 batches x 24 tiles of one column split, 144 tiles at
-    K = 4104 and 150 at K = 4096 stay whole.  int8 splits the 40 and 45 tiles from 33 and 32
-    k-tiles (at most a fifth as many tiles as resident workgroups).  Integer-valued inputs: exact fp32 / int32 sums in any order, so the half
-    outputs are the exact sums rounded once, int8 the low byte, and everything equals the plain
-    kernel's result (tv_hip_gemm_noalloc takes no workspace, hence no stream-K)."""
+    """16-bit and int8 GEMMs with few, long tiles (K = 8192, 4096 and the ragged 8208 and 4104): most are
+    split over K by the multi-stage kernel, tiles summed in segments by several workgroups.  Integer-valued
+    inputs: exact fp32 / int32 sums in any order, so the half outputs are the exact sums rounded once,
+    int8 the low byte, and everything equals the result of whole tiles (tv_hip_gemm_noalloc takes no
+    workspace, hence no split)."""
     lead = (batch,) if batch else ()
     if dt == INT8:
         x = ints(14, lead + (M, K), -128, 127, np.int8)
@@ -472,17 +467,16 @@ def test_direct_load_stream_k_bit_exact(hip, dt, batch, M, K, N):
 
 @pytest.mark.parametrize("dt", [BFLOAT16, FLOAT16, INT8])
 @pytest.mark.parametrize("batch,M,K,N,a_t,b_t", [
-    (0, 2048, 1000, 4096, False, False),  # 512 tiles of 128x128: two per CU, the most on that size
-    (0, 130, 8208, 8000, False, False),   # 126 tiles of 128x128 over 129 k-tiles: split (stream-K)
+    (0, 2048, 1000, 4096, False, False),  # 512 tiles of 128x128: two per CU
+    (0, 130, 8208, 8000, False, False),   # few tiles over 129 k-tiles: split
     (5, 1000, 304, 1096, True, True),     # 360 tiles of 128x128 over a batch, both operands transposed
-    (0, 2100, 520, 4104, False, False),   # 561 tiles of 128x128: runs 153 tiles of 256x256 instead
+    (0, 2100, 520, 4104, False, False),   # 561 tiles of 128x128
     (0, 2104, 520, 4104, True, False),
     (0, 2100, 520, 4104, False, True)],
     ids=["t128-512", "t128-split", "t128-batch-AtBt", "t256-153", "t256-At", "t256-Bt"])
 def test_direct_load_tile_size_exact(hip, dt, batch, M, K, N, a_t, b_t):
-    """16-bit and int8 GEMMs on the direct-load kernels run 128x128 tiles while those fit one round
-    of resident workgroups (two per CU: at most 512 tiles on 256 CUs) and 256x256 tiles above that.
-    Shapes either side of the switch, ragged in M, N and K, with transposed views (int8's 128-row
+    """16-bit and int8 GEMMs on the direct-load kernels, around one round of resident workgroups of 128x128
+    tiles (two per CU: 512 tiles on 256 CUs), ragged in M, N and K, with transposed views (int8's 128-row
     M/N-contiguous layout has its own swizzle; int8 rows whose K is not whole 16-byte chunks are
     copied into padded rows first).  Integer-valued inputs: exact sums in any order, half outputs
     each rounded once, int8 the low byte; a second call gives the same bits."""
@@ -510,10 +504,11 @@ def test_direct_load_tile_size_exact(hip, dt, batch, M, K, N, a_t, b_t):
 @pytest.mark.parametrize("dt", [BFLOAT16, FLOAT16])
 @pytest.mark.parametrize("batch,M,K,N", [(0, 4100, 520, 8200), (0, 4100, 100, 8200), (0, 4100, 50, 8200), (3, 2600, 700, 5000)])
 def test_direct_load_chain_exact(hip, dt, batch, M, K, N):
-    """16-bit GEMMs of at least two 256x256 tiles per CU run the chained persistent kernel (each
-    workgroup's k-loop runs on into its next tile, whose first two k-tiles load during the
-    previous tile's last steps and store): 561 tiles with ragged M, N and K (9 k-tiles, an odd
-    count), K of two and of one k-tile, and 660 tiles over a batch with per-batch B.
+    """16-bit GEMMs of at least two 256x256 tiles per CU, either side of where those tiles are priced below
+    128x128 ones: 660 of them over a batch with per-batch B, which run the chained persistent kernel
+    (each workgroup's k-loop runs on into its next tile, whose first two k-tiles load during the previous
+    tile's last steps and store), and 561 with 9 (an odd count), two and one k-tiles, which run as 2,145 tiles
+    of 128x128; ragged M, N and K.  The chained kernel in every layout: tests/test_kernel_cases_gpu.py.
     Integer-valued inputs in [-2, 2]: the fp32 sums are exact in any order, so the output is each
     exact sum rounded once; a second call gives the same bits."""
     lead = (batch,) if batch else ()
@@ -529,9 +524,9 @@ def test_direct_load_chain_exact(hip, dt, batch, M, K, N):
 @pytest.mark.parametrize("dt", [BFLOAT16, FLOAT16])
 @pytest.mark.parametrize("a_t,b_t", [(True, False), (False, True), (True, True)], ids=["At", "Bt", "AtBt"])
 def test_direct_load_chain_transposed_views(hip, dt, a_t, b_t):
-    """The chained kernel with the other operand layouts, as transposed views consumed through their
-    strides (A M-contiguous, B K-contiguous, or both; every pitch a whole number of 16-byte chunks,
-    so both stay on the direct-load kernels): 561 tiles, ragged M/N, K = 328 (6 k-tiles).
+    """The other operand layouts, as transposed views consumed through their strides (A M-contiguous,
+    B K-contiguous, or both; every pitch a whole number of 16-byte chunks, so both stay on the
+    direct-load kernels): 2,145 tiles of 128x128, ragged M/N, K = 328 (6 k-tiles).
     Integer-valued inputs, exact sums rounded once."""
     M, K, N = 4104, 328, 8200
     x = ints(18, (M, K), -2, 2)

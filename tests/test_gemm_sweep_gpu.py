@@ -2,8 +2,8 @@
 (M, N, K from 1 to a few thousand, log-uniform), batch (none, 1 or 3, B per batch or broadcast)
 and the layout of each operand (row-major, or stored transposed and viewed back).  The router
 sends such calls to every kernel family: the GEMVs (M <= 32), the small-K kernels, the 128x128 and
-256x256 direct-load tiles and their stream-K and chained schedules, the six fp32 tiles, the padded
-row copies of misaligned operands and the element-gather loader.
+256x256 direct-load tiles, the chained schedule and the multi-stage tiles, whole and split over K, the six fp32
+tiles and their stream-K schedule, the 16 x 16-block kernel, the padded row copies of misaligned operands and the element-gather loader.
 
 Inputs are integers in [-3, 3], so every accumulation order gives the same fp32 / int32 sum: fp32
 outputs must equal the exact sum, half outputs the exact sum rounded once, int8 outputs its low

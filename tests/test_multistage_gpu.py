@@ -2,9 +2,11 @@
 split ranges, exact: integer inputs in [-3, 3] make every order of summation give the same fp32 / int32
 sums, so the results equal numpy's product rounded once (int8: its low byte), bit for bit.
 
-The shapes take each tile (32x64 up to 256x128) whole and split, with ragged M, N and K (fewer k-tiles
-than stages; one element past a k-tile), M-contiguous and K-contiguous operands, batches, the rotated
-k-loops of tall calls (many rows of A, one tile column) and the fused epilogue.
+The shapes take the tiles of up to 64 rows whole and split (at 16 bits 32x64 and 64x64, in int8 64x128 as well),
+the two-stage 128x128 tiles and, in fp32, the split two-stage tiles, with ragged M, N and K (fewer k-tiles than stages;
+one element past a k-tile), M-contiguous and K-contiguous operands, batches, rotated k-loops (many rows of A, one
+tile column) and the fused epilogue.  Each instantiation at its edges, the 128x128 and 256x128 multi-stage tiles
+and the rotated 256x128 tile among them: tests/test_kernel_cases_gpu.py.
 """
 import ctypes
 

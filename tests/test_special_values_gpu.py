@@ -27,8 +27,9 @@ CASES = [
     ("fp32_tiles", FLOAT32, 0, 300, 256, 200, False, None, "gemm"),
     ("fp32_stream_k", FLOAT32, 0, 64, 16384, 64, False, None, "gemm"),
     ("fp32_gemv_dot", FLOAT32, 0, 2, 4096, 3000, False, None, "gemm"),
-    ("bf16_256_tiles", BFLOAT16, 0, 512, 512, 520, False, None, "gemm"),
+    ("bf16_256_tiles", BFLOAT16, 0, 512, 512, 520, False, None, "gemm"),  # 32x64 multi-stage tiles, as the next
     ("bf16_128_tiles_bt", BFLOAT16, 0, 300, 1000, 264, True, None, "gemm"),
+    # 2,048 tiles of 128x128; the chained 256x256 tiles: tests/test_kernel_cases_gpu.py
     ("bf16_chained", BFLOAT16, 8, 2048, 256, 2048, False, None, "gemm"),
     ("fp16_small_k", FLOAT16, 16, 1024, 64, 1024, True, None, "gemm"),
     ("bf16_gemv_m1", BFLOAT16, 0, 1, 4096, 4096, False, FLOAT32, "gemv"),

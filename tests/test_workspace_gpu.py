@@ -52,13 +52,18 @@ def _gemm_on(stream, fn, ta, tb):
     return rc, to_storage(tc)
 
 
-# (name, dtype, A shape, B shape, value range): each would use the workspace on a fresh stream.
+# (name, dtype, A shape, B shape, value range): each but the two marked would use the workspace on a fresh
+# stream (tests/test_workspace_lifetime.py checks it).
 CASES = [
     ("bf16_padded_b", BFLOAT16, (64, 512), (512, 260), 3),          # N = 260: B copied into padded rows
     ("bf16_padded_skinny_w", BFLOAT16, (1, 4096), (4096, 129), 2),  # W padded, then the split-K GEMV
     ("bf16_gemv_split_k", BFLOAT16, (8, 4096), (4096, 4096), 2),    # GEMV split-K slots
-    ("fp32_stream_k", FLOAT32, (1024, 1024), (1024, 1024), 3),      # 64 tiles: stream-K slots
-    ("int8_stream_k", INT8, (512, 4096), (4096, 4096), 127),        # 128 tiles of 128x128: split
+    ("fp32_stream_k", FLOAT32, (1024, 1024), (1024, 1024), 3),      # no workspace: 256 tiles of 64x64, whole
+    ("int8_stream_k", INT8, (512, 4096), (4096, 4096), 127),        # no workspace: 256 tiles of 64x128, whole
+    ("fp32_two_stage_split", FLOAT32, (75, 252), (252, 8352), 3),   # stream-K slots
+    ("fp32_split", FLOAT32, (64, 4096), (4096, 64), 3),             # multi-stage tiles split over K
+    ("bf16_split", BFLOAT16, (48, 3712), (3712, 1216), 2),
+    ("int8_split", INT8, (34, 2192), (2192, 1216), 127),
 ]
 
 

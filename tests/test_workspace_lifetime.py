@@ -64,3 +64,13 @@ def test_a_failed_rounded_allocation_is_asked_for_exactly():
     failed = [int(e[1]) for e in r.events if e[0] == "malloc-failed"]
     got = [int(e[2]) for e in r.events if e[0] == "malloc"]
     assert r.rc == 0 and failed == [40 << 20] and got[0] == 4100 * 4096 * 2
+
+
+def test_the_gpu_suites_cases_use_the_workspace():
+    """The calls that tests/test_workspace_gpu.py and tests/test_concurrency_gpu.py run as users of the workspace."""
+    from tests.test_concurrency_gpu import CASES as threads
+    from tests.test_workspace_gpu import CASES as memory
+    calls = [(n, call(*sa, sb[1], dt)) for n, dt, sa, sb, _ in memory] + [(n, call(M, K, N, dt)) for n, dt, M, K, N, _ in threads]
+    for name, line in calls:
+        r, = run(line)
+        assert bool(r.ids("malloc")) == (name not in ("fp32_stream_k", "int8_stream_k")), name
