@@ -296,13 +296,13 @@ static MsPlan ms_plan(const GemmDesc& d, int nk, const MsTile* tiles, const bool
         const int64_t nt = (int64_t)((d.M + t.bm - 1) / t.bm) * ((d.N + t.bn - 1) / t.bn) * d.batch;
         const int64_t slots = (int64_t)cus * t.occ;
         if (nt * (t.bm * t.bn <= 64 * 64 ? 256 : 512) > 0xFFFFFFFFll) continue; // a grid holds fewer than 2^32 threads
-        // us per k-tile with w workgroups in flight.  The two-stage tiles' time grows by half of what a full second
-        // workgroup per CU costs as soon as any CU has two, and with their number (K = 4096, bf16: 258 tiles 56 us,
-        // 512 77).
+        // us per k-tile with w workgroups in flight.  Unsplit plans count a handful of tiles more than CUs as half a
+        // second workgroup on the two-stage tile: bf16 [333,4096]@[4096,11008], 258 tiles, 56 us, 512 of them 77.
         auto step = [&](int64_t w) {
             const double load = (double)((w + cus - 1) / cus - 1);
             if (t.occ == 1 || load <= 0) return t.t1;
-            return t.t1 + (t.tr - t.t1) * (t.s0 < 0 ? 0.5 * load + 0.5 * ((double)w / cus - 1) : load) / (t.occ - 1);
+            const bool handful = !may_split && t.s0 < 0 && w * 16 <= (int64_t)cus * 17;
+            return t.t1 + (t.tr - t.t1) * (handful ? 0.5 : load) / (t.occ - 1);
         };
         auto offer = [&](int64_t wgs, bool split, double k_us, double more) {
             const double us = t.fixed + (k_us > mem ? k_us : mem) + more;
@@ -378,8 +378,8 @@ static int run_ms_cfg(const GemmDesc& d, hipStream_t stream, const MsPlan& plan)
 // 256x256 tiles (bf16 [4096]^3 98 us).
 enum { MS_32x64, MS_64x64, MS_64x128, MS_128x128, MS_256x128, MS_DMA_128, MS_DMA_256, MS_TILES };
 constexpr MsTile kMsTiles[MS_TILES] = {{32, 64, 3, 3.5, 2.0, 1.5, 0.25, 0.43, 3.0, 0.25},  {64, 64, 2, 4.8, 2.6, 1.5, 0.25, 0.43, 3.0, 0.25},
-                                       {64, 128, 1, 5.6, 3.0, 0.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.0, 0.58, 0.58, 5.0, 0.6},
-                                       {256, 128, 1, 6.5, 5.5, 0.0, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.0, 0.67, 1.0, -1, 0},
+                                       {64, 128, 1, 5.0, 3.0, 0.0, 0.42, 0.42, 4.0, 0.35}, {128, 128, 1, 5.0, 4.0, 0.0, 0.58, 0.58, 5.0, 0.6},
+                                       {256, 128, 1, 6.5, 5.5, 0.0, 0.9, 0.9, 8.0, 1.2},   {128, 128, 2, 3.8, 2.5, 0.0, 0.67, 0.95, -1, 0},
                                        {256, 256, 1, 9.0, 7.0, 0.0, 1.3, 1.3, -1, 0}};
 
 // Runs d on the cheapest tile; 1 if that is the 256x256 one, TV_E_NOMEM as run_ms_cfg.  am / bm: the operands' (vector) load modes.

@@ -326,7 +326,8 @@ static int widen(int dt) { return (dt == TV_BFLOAT16 || dt == TV_FLOAT16) ? TV_F
 // so batches of small matrices and thin ones pay for 64 x 64 outputs that they do not have (fp64
 // [100000][4,4]@[4,4] 2,156 us on tiles, 11 here; int32 [10000][8,8]@[8,8] 170, 7; fp64 [1000000,3]@[3,3] 356, 22).
 // Both prices, in us, are fitted to 1,800 random calls (1 to 200,000 matrices of 1 to 500,000 rows or columns, K of 1 to
-// 4096) timed both ways: 2.6 % from the cheaper one on average, 9 of them more than 8 % slower than the tiles.
+// 4096) timed both ways.  The first is the less certain one (how many lines of A and B the L1 keeps), most where
+// latency bounds it, so the tiles are kept unless it is that much less.
 static bool each_output(const GemmDesc& d) {
     const double cus = device_cus(), K = d.K, total = (double)d.batch * d.M * d.N;
     auto tiles = [&](int t) { return (double)(((int64_t)d.M + t - 1) / t) * (double)(((int64_t)d.N + t - 1) / t) * d.batch; };
@@ -346,7 +347,7 @@ static bool each_output(const GemmDesc& d) {
         const double n = tiles(kTile);
         tile = 5.0 + 2.75 * (i64 ? 1.8 : 1.0) * K / kBk * over(n, 0.96 * cus) + 3.9 * n / cus;
     }
-    return each < tile;
+    return (total * mac_us > k_us ? 1.15 : 1.3) * each < tile;
 }
 
 template <typename T, typename R, typename S, bool TILED>

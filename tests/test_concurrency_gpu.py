@@ -28,7 +28,7 @@ pytestmark = pytest.mark.gpu
 CASES = [("bf16_padded_b", BFLOAT16, 64, 512, 260, 3), ("bf16_padded_a", BFLOAT16, 300, 700, 1024, 3),
          ("bf16_padded_skinny_w", BFLOAT16, 1, 4096, 129, 2), ("bf16_gemv_split_k", BFLOAT16, 8, 4096, 4096, 2),
          ("fp32_stream_k", FLOAT32, 1024, 1024, 1024, 3), ("int8_stream_k", INT8, 512, 4096, 4096, 127),
-         ("fp32_two_stage_split", FLOAT32, 75, 252, 8352, 3), ("fp32_split", FLOAT32, 64, 4096, 64, 3),
+         ("fp32_two_stage_split", FLOAT32, 693, 244, 2400, 3), ("fp32_split", FLOAT32, 64, 4096, 64, 3),
          ("bf16_split", BFLOAT16, 48, 3712, 1216, 2), ("int8_split", INT8, 34, 2192, 1216, 127)]
 THREADS = 4
 ITERS = 6

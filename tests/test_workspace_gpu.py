@@ -60,7 +60,7 @@ CASES = [
     ("bf16_gemv_split_k", BFLOAT16, (8, 4096), (4096, 4096), 2),    # GEMV split-K slots
     ("fp32_stream_k", FLOAT32, (1024, 1024), (1024, 1024), 3),      # no workspace: 256 tiles of 64x64, whole
     ("int8_stream_k", INT8, (512, 4096), (4096, 4096), 127),        # no workspace: 256 tiles of 64x128, whole
-    ("fp32_two_stage_split", FLOAT32, (75, 252), (252, 8352), 3),   # stream-K slots
+    ("fp32_two_stage_split", FLOAT32, (693, 244), (244, 2400), 3),   # stream-K slots
     ("fp32_split", FLOAT32, (64, 4096), (4096, 64), 3),             # multi-stage tiles split over K
     ("bf16_split", BFLOAT16, (48, 3712), (3712, 1216), 2),
     ("int8_split", INT8, (34, 2192), (2192, 1216), 127),
