@@ -335,7 +335,8 @@ static bool each_output(const GemmDesc& d) {
     // Lanes on consecutive columns of a row-major B share its lines; rows of fewer than a wave's columns take lines
     // of several rows of A, and a B contiguous along k a line per lane, which the L1 seldom keeps until the next k.
     const bool b_lines = d.sb_n != 1 && d.N > 1, lines = b_lines || d.N < 64;
-    const double k_us = b_lines ? 0.13 : lines ? 0.089 : 0.058, mac_us = lines ? 1.5e-6 : 0.68e-6;
+    const double k_us = b_lines ? 0.13 : lines ? 0.089 : 0.058;
+    const double mac_us = b_lines || d.N < 16 ? 1.5e-6 : lines ? 1.0e-6 : 0.68e-6;
     const double each = 1.9 + K * (total * mac_us > k_us ? total * mac_us : k_us);
     double tile;
     if (d.dtype_a == TV_FLOAT64 && d.dtype_b == TV_FLOAT64) {

@@ -85,7 +85,8 @@ def test_smallest_products(M, K, N, dt, kernel):
     (32, 64, 32, FLOAT64, dict(batch=3000), "gemm_f64_kernel<32,"), (40, 64, 40, FLOAT64, dict(batch=3000), "gemm_f64_kernel<64,"),
     (1000, 1000, 1000, FLOAT64, {}, "gemm_f64_kernel<64,"), (200, 300, 129, FLOAT64, {}, "gemm_f64_kernel<32,"),
     (1000, 600, 1000, INT32, {}, "gemm_simt_kernel"), (128, 512, 65, FLOAT32, dict(db=BFLOAT16, bt=True), "gemm_simt_kernel"),
-    (512, 600, 512, INT16, {}, "gemm_simt_kernel"), (64, 600, 64, INT16, {}, "gemm_each")], ids=str)
+    (512, 600, 512, INT16, {}, "gemm_simt_kernel"), (64, 600, 64, INT16, {}, "gemm_each"),
+    (16, 128, 16, INT32, dict(batch=1000), "gemm_each"), (37, 18, 22, INT32, dict(batch=2988), "gemm_each")], ids=str)
 def test_general_pairs(M, K, N, dt, kw, kernel):
     for r in run(call(M, K, N, dt, **kw), call(M, K, N, dt, **kw, entry="noalloc")):
         assert r.rc == 0 and r.kernel.startswith(kernel)
