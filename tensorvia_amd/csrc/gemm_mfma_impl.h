@@ -545,9 +545,14 @@ __device__ inline void mfma_tile_kloop(const GemmDesc& d, char* smem, int b, int
     u32x4 ra[decltype(la)::NCH];
     u32x4 rb[decltype(lb)::NCH];
     // B fragments of a k-group are held for the whole group; A fragments stream one 16-row block at
-    // a time, one block ahead of the MFMAs that use them.
+    // a time, one block ahead of the MFMAs that use them.  Tile kt+2 is stored over tile kt's stage in the
+    // phase A that follows phase B of kt, with no barrier between the two, so phase B must not read that stage:
+    // k-group 1's A fragments are all read in phase A and held (HOLD).  Tiles whose registers do not hold
+    // them read them in phase B and take a second barrier behind it.
+    constexpr bool HOLD = C::FM <= 4;
     u32x4 fb[C::FN];
     u32x4 fa;
+    u32x4 fh[HOLD ? C::FM : 1];
 
     la.frag_init(lane, wm * C::WM);
     lb.frag_init(lane, wn * C::WN);
@@ -559,8 +564,14 @@ __device__ inline void mfma_tile_kloop(const GemmDesc& d, char* smem, int b, int
     auto kgroup = [&](const char* stage, int kg, const char* nstage, int nkg) {
 #pragma unroll
         for (int i = 0; i < C::FM; ++i) {
-            const u32x4 a_cur = fa;
-            fa = (i + 1 < C::FM) ? a_frag(stage, kg, i + 1) : a_frag(nstage, nkg, 0);
+            const u32x4 a_cur = HOLD && kg == 1 ? fh[HOLD ? i : 0] : fa;
+            if (i + 1 < C::FM) {
+                if (!HOLD || kg == 0) fa = a_frag(stage, kg, i + 1);
+            } else if (!HOLD || kg == 1) {
+                fa = a_frag(nstage, nkg, 0);
+            }
+            if constexpr (HOLD)
+                if (kg == 0) fh[i] = a_frag(nstage, nkg, i);
 #pragma unroll
             for (int j = 0; j < C::FN; ++j) {
                 Op::run(fb[j], a_cur, acc[i][j]);
@@ -583,7 +594,8 @@ __device__ inline void mfma_tile_kloop(const GemmDesc& d, char* smem, int b, int
 
     constexpr int NMF = C::FM * C::FN * Op::kInstr;                  // MFMAs per k-group
     constexpr int NST = decltype(la)::kStores + decltype(lb)::kStores; // LDS stores per tile
-    constexpr int NRD = C::FM * decltype(la)::kFragReads + C::FN * decltype(lb)::kFragReads; // LDS reads per k-group
+    constexpr int NRD = (HOLD ? 2 * C::FM - 1 : C::FM) * decltype(la)::kFragReads + C::FN * decltype(lb)::kFragReads; // LDS reads in phase A
+    constexpr int NRB = (HOLD ? 1 : C::FM) * decltype(la)::kFragReads + C::FN * decltype(lb)::kFragReads;             // and in phase B
     constexpr int NLD = decltype(la)::NCH + decltype(lb)::NCH;        // buffer loads per tile
 
     // k-tiles past kt1 are loaded ahead (zeros past K) but never multiplied.
@@ -623,14 +635,15 @@ __device__ inline void mfma_tile_kloop(const GemmDesc& d, char* smem, int b, int
         lds_barrier();
         // Phase B: MFMAs of k-group 1 of tile kt, reading k-group 0's fragments of tile kt+1.
         kgroup(cur, 1, nxt, 0);
-        if constexpr (NMF >= NRD) {
+        if constexpr (NMF >= NRB) {
 #pragma unroll
-            for (int i = 0; i < NRD; ++i) {
+            for (int i = 0; i < NRB; ++i) {
                 __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(SG_MFMA, NMF - NRD, 0);
+            __builtin_amdgcn_sched_group_barrier(SG_MFMA, NMF - NRB, 0);
         }
+        if constexpr (!HOLD) lds_barrier();
     }
 }
 

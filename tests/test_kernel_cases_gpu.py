@@ -1,7 +1,7 @@
 """Every GEMM kernel instantiation that the dispatch can choose, at sizes ragged in each tile dimension: the calls
 of tests/kernel_cases.py, whose kernels tests/test_kernel_cases.py checks.  Integer inputs in [-2, 2] (sums below
 2^24): every order of summation gives the same fp32 / int32 sum, so results equal the 64-bit product rounded once
-(int8: its low byte), bit for bit; two calls in a row, the second with the counters the first left."""
+(int8: its low byte), bit for bit; calls in a row, each after the first with the counters the one before left."""
 import ctypes
 
 import pytest
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 NAMES = {BFLOAT16: "bf16", FLOAT16: "fp16", FLOAT32: "fp32", INT8: "int8"}
 
 
-def _run(dt, case):
+def _run(dt, case, calls=2):
     _, _, (b, M, K, N), at, bt, act = case
     tdt = tv.tv_to_torch(dt)
     g = torch.Generator(device="cuda")
@@ -41,7 +41,7 @@ def _run(dt, case):
     if act:
         ep.act, ep.bias, ep.sbias_n = tv.ACT_RELU, bias.data_ptr(), 1
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    for _ in range(2):
+    for _ in range(calls):
         c.fill_(7)
         tv.check(tv.lib().tv_hip_gemm_ex(ctypes.byref(args), ctypes.byref(ep), s) if act else tv.lib().tv_hip_gemm(ctypes.byref(args), s))
         torch.cuda.synchronize()
@@ -86,3 +86,12 @@ def test_kernel_exact_fp16(hip, case):
                                      for dt in (BFLOAT16, FLOAT32) for c in CASES[dt] if not c[5]])
 def test_kernel_special_values(hip, dt, case):
     _special(dt, case)
+
+
+@pytest.mark.parametrize("dt,case", [pytest.param(dt, c, id=f"{NAMES[dt]}-{case_id(c)}") for dt in (BFLOAT16, INT8, FLOAT32)
+                                     for c in CASES[dt] if "mfma" in c[0] and c[5]])
+def test_register_staged_kloop_repeated(hip, dt, case):
+    """The k-loop that stages its operands through registers, 150 calls of each: a wave one k-tile ahead must not
+    store over fragments that another wave has still to read (without that order [6][92,628]@[628,3152] was wrong in one
+    fp32 call of forty)."""
+    _run(dt, case, 150)
