@@ -115,7 +115,8 @@ typedef struct tv_gemm_args {
 
 /* General batched matmul.  Routes M <= 8 shapes to the GEMV kernels when they serve the
  * dtype/layout, and 9 <= M <= 32 to the matrix-core GEMV (16-bit W up to 32 rows, int8 W up to 16,
- * whole 128-byte strips), everything else to the MFMA GEMM kernels (or the SIMT slow path). */
+ * whole 128-byte strips), everything else to the GEMM kernels of its dtype pair
+ * (fp32, 16-bit, int8, fp64: matrix cores; the rest: SIMT). */
 int tv_hip_gemm(const tv_gemm_args* args, void* hip_stream);
 
 /* Activations of the fused epilogue (the reference's ops::Relu / Silu / Sigmoid / Tanh). */

@@ -7,7 +7,7 @@
 // What bounds it: the fp64 matrix rate (as high as the vector one, 64 FMAs per CU and cycle), if the
 // operands reach it.  A vector kernel would be LDS-bound: a 4 x 4 block per thread reads 64 bytes for
 // 16 FMAs, twice what LDS delivers in the FMAs' time.  The matrix instruction needs one A and one B
-// value per lane for 16 FMAs, and a wave's 32 x 32 block (2 x 2 instructions) uses each twice.
+// value per lane for 16 FMAs, and a wave's 32 x 16 block (2 x 1 instructions) uses each of B's twice.
 //  * A workgroup computes TILE x TILE outputs, TILE = 64 (8 waves of 32 x 16, two per SIMD) or 32 (4
 //    waves of 16 x 16).
 //  * 32 k of each operand per step, in LDS rows of one output row or column each.  Two LDS stages and

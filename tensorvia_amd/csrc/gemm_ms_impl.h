@@ -389,7 +389,7 @@ static int run_modes_ms(const GemmDesc& d, hipStream_t stream, int group_m, int 
     const int nk = (d.K + 128 / (int)sizeof(T) - 1) / (128 / (int)sizeof(T));
     // Layouts: 32 rows K-contiguous only; 64 rows M/N-contiguous at 16 bits only (DmaOperand).
     const bool r64a = am == LOAD_KCONTIG || !kI8, r64b = bm == LOAD_KCONTIG || !kI8;
-    // Two shapes outside the prices, measured on 450 calls of 16,384 to 131,072 rows or columns, K of 64 to 8192:
+    // Two shapes outside the prices, measured on 507 calls of up to 131,072 rows or columns, K of 64 to 8192:
     //  * Tall: A streamed in rows of whole 4 KB by tiles of one column (N above 64, in batches from 96), at least
     //    one 256x128 tile per CU, up to 512 MB of A: 256x128, rotated.  us, 256x128 rotated / 128x128: bf16
     //    [65536,2048]@[2048,128] 42.2 / 49.6, [131072,2048]@[2048,72] 114 / 132, [65536,4096]@[4096,128] 107 / 128,
